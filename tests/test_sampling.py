@@ -153,3 +153,41 @@ def test_sampling_against_oracle_state():
     assert obs[~nz].sum() == 0
     stat = float(((obs[nz] - shots * p[nz]) ** 2 / (shots * p[nz])).sum())
     assert chi2.sf(stat, int(nz.sum()) - 1) > 1e-6, stat
+
+
+def _uniforms(seed, bsz, shots):
+    """The documented uniforms: splitmix64(seed ^ splitmix64(row * shots + shot)), top 53 bits."""
+    m = (1 << 64) - 1
+
+    def mix(x):
+        x = (x + 0x9E3779B97F4A7C15) & m
+        x = ((x ^ (x >> 30)) * 0xBF58476D1CE4E5B9) & m
+        x = ((x ^ (x >> 27)) * 0x94D049BB133111EB) & m
+        return x ^ (x >> 31)
+
+    return np.array([(mix(seed ^ mix(w)) >> 11) / 2.0 ** 53 for w in range(bsz * shots)]).reshape(bsz, shots)
+
+
+@gpu
+@pytest.mark.parametrize("n", [1, 5, 6, 7, 11, 12, 13, 15])
+@pytest.mark.parametrize("holes", [False, True])
+def test_shots_invert_the_cumulative_distribution(n, holes):
+    """Every shot is the amplitude whose slice of the cumulative |psi|^2 holds its uniform, to the rounding of the
+    probabilities (each within 2^-23 of itself in float32, so their sums within 2^-23 of the total; four times
+    that is allowed); blocks and segments cut short, whole and empty."""
+    bsz, shots, seed = 3, 500, 12345
+    q, v = _random_state_dev(n, bsz, 40 + n)
+    if holes:                       # mass in a few places only: empty segments and blocks between them
+        keep = np.zeros(2 ** n, dtype=bool)
+        keep[np.random.default_rng(n).choice(2 ** n, max(1, 2 ** n // 50), replace=False)] = True
+        v = v * keep
+        q.set_states(torch.tensor(v, dtype=torch.complex64, device="cuda"))
+    v = q.get_states_1d().cpu().numpy().astype(np.complex128)
+    idx = tq.sample_indices(q, shots, seed=seed).cpu().numpy()
+    u = _uniforms(seed, bsz, shots)
+    for b in range(bsz):
+        p = np.abs(v[b]) ** 2
+        cum = np.cumsum(p)
+        t, tol = u[b] * cum[-1], 4 * 2.0 ** -23 * cum[-1]
+        assert (p[idx[b]] > 0).all()
+        assert (t <= cum[idx[b]] + tol).all() and (t >= cum[idx[b]] - p[idx[b]] - tol).all()
