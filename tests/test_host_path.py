@@ -1,0 +1,124 @@
+"""The native recording and plan keys (csrc/tqsv_host.cpp) against the general Python path they stand in for."""
+import itertools
+
+import numpy as np
+import pytest
+import torch
+
+import torchquantum_amd as tq
+import torchquantum_amd.functional as tqf
+from torchquantum_amd import _native as N
+from torchquantum_amd import engine as E
+from torchquantum_amd import operator as op
+
+NQ, BSZ = 5, 3
+WIRES = [0, 4, 5, -1, True, np.int64(2), [1], (2,), [0, 3], (3, 0), [2, 2], [0, 9], [1, 2, 3], np.array([1, 4]), []]
+PARAMS = [None, 0.3, [0.1, 0.2, 0.3], torch.tensor(0.4), torch.rand(1), torch.rand(BSZ), torch.rand(1, 1),
+          torch.rand(BSZ, 1), torch.rand(1, 3), torch.rand(BSZ, 3), torch.rand(3, BSZ).T, torch.rand(1, 1).double(),
+          torch.rand(1, 1).to(torch.complex64), torch.rand(1, 1, requires_grad=True), torch.rand(1, 2)]
+
+
+def _outcome(f):
+    """What a recording leaves behind: the tape entries, or the exception's type and text."""
+    q = tq.QuantumDevice(n_wires=NQ, bsz=BSZ, device="cpu")
+    try:
+        f(q)
+    except Exception as e:      # noqa: BLE001 -- compared with the other path's
+        return type(e), str(e)
+    return [(o.name, o.wires, [type(w) for w in o.wires], o.inverse, o.version, o.conj, o.nonunitary,
+             None if o.params is None else (o.params.dtype, tuple(o.params.shape), o.params.tolist())) for o in q._tape]
+
+
+@pytest.mark.parametrize("name", ["rx", "u3", "hadamard", "cnot", "crx", "toffoli", "multicnot", "swap", "i"])
+def test_gates_as_the_general_path_records_them(name):
+    params = PARAMS if name in ("rx", "u3", "crx") else [None, torch.rand(1, 1)]
+    for w, p, inv in itertools.product(WIRES, params, (False, True, 1)):
+        got = _outcome(lambda q: tqf.func_name_dict[name](q, w, params=p, inverse=inv))
+        want = _outcome(lambda q: tqf.gate_wrapper(name, q, w, p, inverse=inv))
+        assert got == want, (name, w, p, inv)
+
+
+def _ops():
+    """Operators in every state a call can meet them in, and whether the call itself has to run."""
+    a, b, c, d, e, f = (op.RX(has_params=True, trainable=True) for _ in range(6))
+    b = op.RX()
+    b.params = torch.rand(BSZ, 1)                    # a plain tensor instead of a parameter
+    c.register_forward_pre_hook(lambda m, i: None)
+    d.forward = lambda q_device, wires=None: tqf.rz(q_device, wires, params=torch.ones(1, 1))
+    e.func = tqf.ry
+    f.inverse = True
+    g = op.RX()
+    g.params = torch.rand(1)                         # one dimension: the call reshapes it
+    return [a, b, c, d, e, f, g, op.Hadamard(), op.RX(), op.I()]
+
+
+class _Doubled(op.RX):
+    def forward(self, q_device, wires=None):
+        super().forward(q_device, wires=wires)
+        super().forward(q_device, wires=wires)
+
+
+@pytest.mark.parametrize("record_op", [False, True])
+def test_layers_as_the_operator_calls_record_them(record_op):
+    for o in _ops() + [_Doubled(has_params=True), op.CNOT()]:
+        for w in (2, [2], [0, 3], 7, [1, 1]):
+            seen = []
+            for each in (True, False):
+                torch.manual_seed(0)
+
+                def rec(q):
+                    q.record_op = record_op
+                    op.apply_each(q, [o], [w]) if each else o(q, wires=w)
+                    seen.append((list(q.op_history), o.wires))
+                seen.append(_outcome(rec))
+            assert seen[:len(seen) // 2] == seen[len(seen) // 2:], (o, w)
+
+
+def test_hooks_run():
+    layer = tq.Op1QAllLayer(op.RY, 4, has_params=True, trainable=True)
+    ran = []
+    layer.ops_all[2].register_forward_hook(lambda m, i, o: ran.append(m))
+    layer(tq.QuantumDevice(n_wires=4, device="cpu"))
+    assert ran == [layer.ops_all[2]]
+    h = torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: ran.append(m))
+    try:
+        layer(tq.QuantumDevice(n_wires=4, device="cpu"))
+    finally:
+        h.remove()
+    assert len([m for m in ran if isinstance(m, op.RY)]) == 1 + 4 + 1
+
+
+def _python_key(tape):
+    return tuple((o.name, o.wires, o.inverse, o.conj, None if o.params is None else
+                  ("m", o.params.shape) if o.params.is_complex() else
+                  (o.params.shape, o.params.requires_grad, o.params.is_cuda, o.params.dtype)) for o in tape)
+
+
+def test_structure_is_equal_exactly_where_the_plan_is():
+    one = [E.TapeOp(nm, w, p, inv, 0, cj) for nm in ("rx", "r", "xr") for w in ((0,), (1,), (0, 1))
+           for p in (None, torch.rand(1, 1), torch.rand(1, 1, requires_grad=True), torch.rand(2, 1),
+                     torch.rand(1, 1).double(), torch.rand(1, 2, 2).to(torch.complex64),
+                     torch.rand(1, 2, 2, requires_grad=True).to(torch.complex64), torch.rand(2, 2).to(torch.complex64))
+           for inv in (False, True) for cj in (False, True)]
+    tapes = [[]] + [[o] for o in one] + [[one[0], o] for o in one[::7]] + [[o, one[0]] for o in one[::7]]
+    keys = [(N.host().structure(t), _python_key(t)) for t in tapes]
+    for a, b in itertools.combinations(keys, 2):
+        assert (a[0] == b[0]) == (a[1] == b[1])
+
+
+def test_stale_parameters_and_pointers():
+    p = [torch.rand(3, 2), torch.rand(1, 2), torch.rand(4, 6)[:, 1:5:2], torch.rand(2, 3).T]
+    tape = [E.TapeOp("u2", (0,), t, False, t._version) for t in p] + [E.TapeOp("hadamard", (0,), None)]
+    assert N.host().stale(tape) == -1
+    out = np.zeros((4, 3), dtype=np.int64)
+    N.host().pointers(tape, np.array([3, 0, 2, 1], dtype=np.int32), out)
+    want = [[t.data_ptr(), t.stride(0) if t.shape[0] > 1 else 0, t.stride(1)] for t in (p[3], p[0], p[2], p[1])]
+    assert out.tolist() == want
+    p[2].add_(1)
+    assert N.host().stale(tape) == 2
+    for bad in (np.array([4], dtype=np.int32), np.array([-1], dtype=np.int32), np.array([0], dtype=np.int64)):
+        with pytest.raises(ValueError):
+            N.host().pointers(tape, bad, out)
+    for f in (N.host().stale, N.host().structure):
+        with pytest.raises(TypeError):
+            f([None])

@@ -113,6 +113,24 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The host extension (csrc/tqsv_host.cpp): recording, plan keys, parameter pointers."""
+    global _host
+    if _host is None:
+        try:
+            from . import _tqhost
+        except ImportError as e:
+            raise NativeError("torchquantum_amd/_tqhost.so is not built; run `python -m torchquantum_amd.csrc.build`") \
+                from e
+        from .engine import TapeOp
+        _tqhost.bind(TapeOp)
+        _host = _tqhost
+    return _host
+
+
 def exported_symbols():
     L = lib()
     return {n for n in SIGNATURES if getattr(L, n, None) is not None}
@@ -131,7 +149,8 @@ def call(name: str, *args):
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Raw handle of the current stream of the tensor's device."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def require_gpu(t: torch.Tensor, what: str = "tensor"):

@@ -12,6 +12,7 @@
 """
 from __future__ import annotations
 
+import functools
 from typing import List, Sequence, Tuple
 
 import numpy as np
@@ -47,22 +48,24 @@ class CircuitFunction(torch.autograd.Function):
         c = payload.c
         lam_in = gout.to(torch.complex64).reshape(out.shape).contiguous()
         grad, lam = E.adjoint(c, out, lam_in, ctx.pool, need_input_grad=ctx.needs_input_grad[1])
-        gsum = None            # batch-row sums for parameters shared by all rows, one reduction
+        # parameters shared by all rows take the sums over the rows; all
+        # gradients are slices of two buffers, cut in one call each
+        need = ctx.needs_input_grad[2:]
+        shared = rows = None
+        if any(n and s for n, s in zip(need, c.param_shared)):
+            shared = grad.sum(0, keepdim=True)[:, :c.n_slots].split(c.param_widths, 1)
+        if any(n and not s for n, s in zip(need, c.param_shared)):
+            rows = grad[:, :c.n_slots].split(c.param_widths, 1)
         grads: List = []
-        for j, ti in enumerate(payload.param_idx):
-            if not ctx.needs_input_grad[2 + j]:
+        for j, wanted in enumerate(need):
+            if not wanted:
                 grads.append(None)
                 continue
-            op = payload.tape[ti]
-            off = c.param_offsets[ti]
-            P = op.n_params()
-            if op.params.shape[0] == 1:
-                if gsum is None:
-                    gsum = grad.sum(0, keepdim=True)
-                g = gsum[:, off:off + P]
-            else:
-                g = grad[:, off:off + P]
-            grads.append(g.reshape(op.params.shape).to(op.params.dtype))
+            g = shared[j] if c.param_shared[j] else rows[j]
+            if not c.param_plain[j]:
+                p = payload.tape[payload.param_idx[j]].params
+                g = g.reshape(p.shape).to(p.dtype)
+            grads.append(g)
         gstate = lam if ctx.needs_input_grad[1] else None
         return (None, gstate, *grads)
 
@@ -135,6 +138,10 @@ class ExpvalZAll(torch.autograd.Function):
         return lam.reshape(ctx.shape), None
 
 
+_PHASE = np.array([1, 1j, -1, -1j])      # i^{nY}
+
+
+@functools.lru_cache(maxsize=4096)
 def pauli_masks(obs: str, n: int) -> Tuple[int, int, int]:
     """(x mask, z mask, number of Y) of a Pauli string; char k <-> wire k."""
     obs = obs.upper()
@@ -179,7 +186,7 @@ class ExpvalPauli(torch.autograd.Function):
     def backward(ctx, g: torch.Tensor):
         (st,) = ctx.saved_tensors
         n, xs, zs, nys, shape = ctx.meta
-        phase = torch.tensor([(1j) ** (k % 4) for k in nys], dtype=torch.complex64, device=st.device)
+        phase = E.upload(_PHASE[np.array(nys, dtype=np.int64) % 4].astype(np.complex64), st.device)
         coef = 2.0 * g.to(torch.complex64) * phase[None, :]
         lam = _pauli_apply(st, n, xs, zs, coef)
         return lam.reshape(shape), None, None, None, None
@@ -200,11 +207,11 @@ class ExpvalPauliSum(torch.autograd.Function):
         bsz = state.shape[0]
         st = _rows(state, bsz)
         if not ctx.needs_input_grad[0]:
-            c = torch.tensor(coef, dtype=torch.float32, device=st.device)
+            c = E.upload(np.array(coef, dtype=np.float32), st.device)
             return _expval_terms(st, n, xs, zs) @ c
         T = len(xs)
-        cw = torch.tensor([2.0 * float(c) * (1j) ** (k % 4) for c, k in zip(coef, nys)], dtype=torch.complex64,
-                          device=st.device)
+        cw = E.upload((2.0 * np.array(coef, dtype=np.float64) * _PHASE[np.array(nys, dtype=np.int64) % 4])
+                      .astype(np.complex64), st.device)
         w = torch.empty_like(st)
         dot = torch.empty(bsz, dtype=torch.float32, device=st.device)
         nws = int(N.lib().tqsv_pauli_sum_grad_workspace_floats(bsz, n))

@@ -20,6 +20,7 @@ import numpy as np
 import torch
 import torch.nn as nn
 
+from . import _native as N
 from . import engine as E
 from .autograd import run_tape
 from .macro import C_DTYPE
@@ -84,9 +85,9 @@ class QuantumDevice(nn.Module):
                 self._sv = self._zero_state()
             return
         tape, self._tape = self._tape, []
-        for op in tape:
-            if op.params is not None and op.params._version != op.version:
-                raise RuntimeError(f"parameter of gate '{op.name}' was modified in place after the gate call")
+        i = N.host().stale(tape)
+        if i >= 0:
+            raise RuntimeError(f"parameter of gate '{tape[i].name}' was modified in place after the gate call")
         dev = self._sv_device()
         if self._sv is None:
             dummy = torch.empty(0, dtype=C_DTYPE, device=dev)

@@ -656,47 +656,58 @@ class _HostMirror:
 _MIRROR = _HostMirror()
 
 
-class _PinnedRing:
-    """Matrix-pool uploads through a fixed ring of pinned host buffers.
+_TORCH_DTYPE = {np.dtype(np.complex64): torch.complex64, np.dtype(np.float32): torch.float32,
+                np.dtype(np.int64): torch.int64}
 
-    A flush copies its pool host -> device asynchronously, so the host can run
-    ahead of the GPU.  A slot is refilled only after the copy that last used
-    it has completed (its event), which bounds how far ahead the host runs;
-    buffers grow on demand and are never freed, so steady-state flushes make
-    no pinned allocations."""
+
+class _PinnedRing:
+    """Host -> device uploads through a fixed ring of pinned host buffers.
+
+    A flush copies its matrix pool (and an expectation its coefficients)
+    asynchronously, so the host can run ahead of the GPU.  A slot is refilled
+    only after the copy that last used it has completed (its event), which
+    bounds how far ahead the host runs; buffers grow on demand and are never
+    freed, so steady-state flushes make no pinned allocations."""
 
     SLOTS = 8
 
     def __init__(self):
-        self.slots: List[Optional[tuple]] = [None] * self.SLOTS
+        self.slots: List[Optional[tuple]] = [None] * self.SLOTS     # (pinned bytes, their numpy view, event)
         self.i = 0
         self.lock = threading.Lock()
 
+    @staticmethod
+    def _slot(cap: int) -> tuple:
+        buf = torch.empty(cap, dtype=torch.uint8, pin_memory=True)
+        return buf, buf.numpy(), None
+
     def upload(self, host: np.ndarray, device: torch.device) -> torch.Tensor:
-        flat = np.ascontiguousarray(host, dtype=np.complex64).reshape(-1)
-        n = flat.size
+        raw = np.ascontiguousarray(host).reshape(-1).view(np.uint8)
+        n = raw.size
         with self.lock:
             i = self.i
             self.i = (i + 1) % self.SLOTS
-            buf, ev = self.slots[i] if self.slots[i] is not None else (None, None)
-            if ev is not None:
-                ev.synchronize()
-            if buf is None or buf.numel() < n:
-                cap = max(n, 2 * (buf.numel() if buf is not None else 0), 4096)
-                buf = torch.empty(cap, dtype=torch.complex64, pin_memory=True)
+            slot = self.slots[i]
+            if slot is not None and slot[2] is not None:
+                slot[2].synchronize()
+            if slot is None or slot[0].numel() < n:
+                cap = max(n, 2 * (slot[0].numel() if slot is not None else 0), 1 << 15)
+                slot = self._slot(cap)
                 # the first use fills every empty slot too, so that later
                 # flushes make no pinned allocation (slots that are still
                 # empty have no copy in flight)
                 for j in range(self.SLOTS):
                     if j != i and self.slots[j] is None:
-                        self.slots[j] = (torch.empty(cap, dtype=torch.complex64, pin_memory=True), None)
-            buf[:n].numpy()[:] = flat
-            out = torch.empty(n, dtype=torch.complex64, device=device)
+                        self.slots[j] = self._slot(cap)
+            buf, view, ev = slot
+            view[:n] = raw
+            out = torch.empty(n, dtype=torch.uint8, device=device)
             out.copy_(buf[:n], non_blocking=True)
-            ev = torch.cuda.Event()
+            if ev is None:
+                ev = torch.cuda.Event()
             ev.record(torch.cuda.current_stream(device))
-            self.slots[i] = (buf, ev)
-        return out.reshape(host.shape)
+            self.slots[i] = (buf, view, ev)
+        return out.view(_TORCH_DTYPE[host.dtype]).reshape(host.shape)
 
 
 _RINGS: Dict[torch.device, _PinnedRing] = {}
@@ -714,7 +725,12 @@ def _check_dev_layout():
         _DEV_LAYOUT_OK = True
 
 
-def _upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
+def upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
+    """Copy of a complex64, float32 or int64 array on the device, enqueued on
+    the current stream without waiting for the work already there (a copy
+    from pageable memory, as ``torch.tensor(..., device=)`` makes, waits)."""
+    if device.type != "cuda" or host.size == 0:
+        return torch.from_numpy(host).to(device)
     if device.index is None:
         device = torch.device("cuda", torch.cuda.current_device())
     ring = _RINGS.get(device)
@@ -1313,6 +1329,13 @@ class Compiled:
         # tape ops with real parameters, and whether any of them is trainable
         # (both fixed by the structure key, which holds shapes and requires_grad)
         self.param_idx = [i for i, op in enumerate(tape) if op.params is not None and not op.is_matrix_param]
+        # how backward() hands out the gradient columns: widths in order, and
+        # per parameter whether all rows share it and whether a [1 or bsz, P]
+        # float32 slice is already its gradient
+        self.param_widths = [tape[i].n_params() for i in self.param_idx]
+        self.param_shared = [tape[i].params.shape[0] == 1 for i in self.param_idx]
+        self.param_plain = [tape[i].params.dim() == 2 and tape[i].params.dtype == torch.float32
+                            for i in self.param_idx]
         self.any_param_grad = any(tape[i].params.requires_grad for i in self.param_idx)
         kops = lower(tape, n, bsz, self.param_offsets)
         if opts.mode == "fused" and opts.fusion_width >= 2:
@@ -1387,6 +1410,8 @@ class Compiled:
                 members.append(rec)
         self.dev_members = np.concatenate(members) if members else np.zeros(0, dtype=DEV_MEMBER)
         self.dev_deriv_ops = np.array(deriv_ops, dtype=np.int64)
+        self.dev_param_mem = np.array(self.dev_param_mem, dtype=np.int64)
+        self.dev_param_tape = np.array(self.dev_param_tape, dtype=np.int32)
         self.dev_tail = (self.dev_ops.nbytes + self.dev_members.nbytes) // 8     # complex64 elements
         # every parameterised op built on the GPU: the host part of the pool
         # depends on the plan only and is built once
@@ -1596,7 +1621,7 @@ class Compiled:
         host = self.pool_host(tape, with_grad, with_adj)
         if torch.device(self.device).type != "cuda":
             return torch.from_numpy(host).to(self.device)
-        pool = _upload(host, torch.device(self.device))
+        pool = upload(host, torch.device(self.device))
         if len(self.dev_ops):
             _check_dev_layout()
             base = pool.data_ptr() + 8 * self.pool_len
@@ -1613,10 +1638,11 @@ class Compiled:
                 ops = ops.copy()
                 ops["flags"][self.dev_deriv_ops] |= DGF_DERIV
             mem = self.dev_members.copy()
-            ps = [tape[t].params for t in self.dev_param_tape]
-            mem["params"][self.dev_param_mem] = [p.data_ptr() for p in ps]
-            mem["rstride"][self.dev_param_mem] = [p.stride(0) if p.shape[0] > 1 else 0 for p in ps]
-            mem["cstride"][self.dev_param_mem] = [p.stride(1) for p in ps]
+            at = np.empty((len(self.dev_param_mem), 3), dtype=np.int64)
+            N.host().pointers(tape if type(tape) is list else list(tape), self.dev_param_tape, at)
+            mem["params"][self.dev_param_mem] = at[:, 0]
+            mem["rstride"][self.dev_param_mem] = at[:, 1]
+            mem["cstride"][self.dev_param_mem] = at[:, 2]
             tail = (ops, mem)
         if self._static_host is not None:
             host = np.empty(self.pool_len + self.dev_tail, dtype=np.complex64)
@@ -1775,18 +1801,7 @@ _plan_cache: Dict[tuple, Compiled] = {}
 
 
 def structure_key(tape: Sequence[TapeOp], n: int, bsz: int, opts: EngineOptions, device) -> tuple:
-    items = []
-    add = items.append
-    for op in tape:
-        p = op.params
-        if p is None:
-            ps = None
-        elif p.is_complex():
-            ps = ("m", p.shape)                 # torch.Size: a tuple (hash and equality)
-        else:
-            ps = (p.shape, p.requires_grad, p.is_cuda, p.dtype)
-        add((op.name, op.wires, op.inverse, op.conj, ps))
-    return (n, bsz, opts.key(), str(device), tuple(items))
+    return (n, bsz, opts.key(), str(device), N.host().structure(tape if type(tape) is list else list(tape)))
 
 
 def compile_tape(tape: Sequence[TapeOp], n: int, bsz: int, opts: EngineOptions, device) -> Compiled:

@@ -17,6 +17,7 @@ import numpy as np
 import torch
 
 from .. import gates as G
+from .. import _native as N
 from ..engine import TapeOp
 from ..macro import C_DTYPE, F_DTYPE
 
@@ -126,38 +127,18 @@ def _make_gate(name: str):
 
     def gate(q_device, wires, params=None, n_wires=None, static=False, parent_graph=None, inverse=False,
              comp_method="bmm"):
-        # fast path, same checks as _record: a fixed-width gate on int wires
-        # with no parameter or a real [rows, P] tensor, no op history
+        # the plain form (a fixed-width gate on int wires, no parameter or a
+        # real [rows, P] tensor, no op history) is recorded natively
         if plain and comp_method == "bmm" and not getattr(q_device, "record_op", False):
-            tw = type(wires)
-            ws = None
-            if tw is int:
-                ws = (wires,)
-            elif tw is list or tw is tuple:
-                ws = tuple(wires)
-                for w in ws:
-                    if type(w) is not int:
-                        ws = None
-                        break
-            if ws is not None and len(ws) == nw and (nw == 1 or len(set(ws)) == nw):
-                n = q_device.n_wires
-                ok = True
-                for w in ws:
-                    if w < 0 or w >= n:
-                        ok = False
-                        break
-                if ok:
-                    if npar == 0:
-                        q_device._push(TapeOp(cname, ws, None, bool(inverse), 0))
-                        return
-                    if (type(params) is torch.Tensor or isinstance(params, torch.Tensor)) and params.dim() == 2 \
-                            and params.shape[-1] == npar and not params.is_complex():
-                        q_device._push(TapeOp(cname, ws, params, bool(inverse), params._version))
-                        return
+            op = N.host().make(cname, nw, npar, wires, params, inverse, q_device.n_wires)
+            if op is not None:
+                q_device._push(op)
+                return
         _record(name, cname, spec, q_device, wires, params, inverse, comp_method)
 
     gate.__name__ = name
     gate.__qualname__ = name
+    gate.plain_spec = (cname, nw, npar) if plain else None
     gate.__doc__ = f"Apply the {name} gate (torchquantum.functional.{name} semantics)."
     return gate
 

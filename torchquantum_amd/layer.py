@@ -25,8 +25,7 @@ class Op1QAllLayer(QuantumModule):
 
     @static_support
     def forward(self, q_device):
-        for k in range(self.n_wires):
-            self.ops_all[k](q_device, wires=k)
+        op.apply_each(q_device, list(self.ops_all)[:self.n_wires], range(self.n_wires))
 
 
 class Op2QAllLayer(QuantumModule):
@@ -47,11 +46,12 @@ class Op2QAllLayer(QuantumModule):
 
     @static_support
     def forward(self, q_device):
-        for k in range(len(self.ops_all)):
-            wires = [k, (k + self.jump) % self.n_wires]
-            if self.wire_reverse:
-                wires.reverse()
-            self.ops_all[k](q_device, wires=wires)
+        n, jump = self.n_wires, self.jump
+        if self.wire_reverse:
+            wires = [[(k + jump) % n, k] for k in range(len(self.ops_all))]
+        else:
+            wires = [[k, (k + jump) % n] for k in range(len(self.ops_all))]
+        op.apply_each(q_device, self.ops_all, wires)
 
 
 class EntanglePairwise(QuantumModule):
@@ -68,14 +68,9 @@ class EntanglePairwise(QuantumModule):
 
     @static_support
     def forward(self, q_device):
-        k = 0
-        for start in (0, 1):
-            for i in range(start, self.n_wires - 1, 2):
-                wires = [i, i + 1]
-                if self.wire_reverse:
-                    wires.reverse()
-                self.ops_all[k](q_device, wires=wires)
-                k += 1
+        pairs = [[i + 1, i] if self.wire_reverse else [i, i + 1]
+                 for start in (0, 1) for i in range(start, self.n_wires - 1, 2)]
+        op.apply_each(q_device, self.ops_all, pairs)
 
 
 class LayerTemplate0(QuantumModule):
@@ -147,5 +142,4 @@ class RandomLayer(QuantumModule):
 
     @static_support
     def forward(self, q_device):
-        for o, w in zip(self.op_list, self.op_wires):
-            o(q_device, wires=w)
+        op.apply_each(q_device, self.op_list, self.op_wires)

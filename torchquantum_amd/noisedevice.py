@@ -27,7 +27,7 @@ Deliberate differences from the reference (both are errors there):
 """
 from __future__ import annotations
 
-import dataclasses
+import functools
 from typing import List, Optional, Sequence, Union
 
 import numpy as np
@@ -35,6 +35,7 @@ import torch
 import torch.nn as nn
 
 from . import engine as E
+from .autograd import _PHASE, pauli_masks
 from .device import QuantumDevice, _default_device
 
 C_DTYPE = torch.complex64
@@ -50,7 +51,7 @@ def superoperator(kraus: Sequence[np.ndarray]) -> np.ndarray:
     d = ks[0].shape[0]
     if any(k.shape != (d, d) for k in ks):
         raise ValueError("Kraus operators must be square and of one size")
-    return sum(np.kron(k, np.conj(k)) for k in ks)
+    return sum((k[:, None, :, None] * np.conj(k)[None, :, None, :]).reshape(d * d, d * d) for k in ks)
 
 
 def amplitude_damping_kraus(gamma: float) -> List[np.ndarray]:
@@ -120,7 +121,8 @@ class NoiseDevice(nn.Module):
         """A gate U on wires W: U on the row wires, conj(U) on the column wires."""
         n = self.n_wires
         self.reg._push(op)
-        self.reg._push(dataclasses.replace(op, wires=tuple(w + n for w in op.wires), conj=not op.conj))
+        self.reg._push(E.TapeOp(op.name, tuple([w + n for w in op.wires]), op.params, op.inverse, op.version,
+                                not op.conj, op.nonunitary))
 
     def flush(self, options: Optional[E.EngineOptions] = None):
         self.reg.flush(options)
@@ -129,38 +131,42 @@ class NoiseDevice(nn.Module):
     def kraus(self, wires: Union[int, Sequence[int]], kraus_ops: Sequence[np.ndarray]):
         """rho -> sum_k K_k rho K_k^dagger on ``wires`` (K_k: 2^k x 2^k, wires[0]
         the most significant bit, as for the gates)."""
+        self._channel(wires, superoperator(kraus_ops))
+
+    def _channel(self, wires: Union[int, Sequence[int]], S: np.ndarray):
+        """Record a channel given as its superoperator.  The matrix stays on
+        the host, where the flush builds its matrix pool."""
         ws = [int(wires)] if isinstance(wires, (int, np.integer)) else [int(w) for w in wires]
         n = self.n_wires
         if len(set(ws)) != len(ws) or any(not 0 <= w < n for w in ws):
             raise ValueError(f"bad wires {ws} for {n} wires")
-        S = superoperator(kraus_ops)
         if S.shape[0] != 1 << (2 * len(ws)):
             raise ValueError(f"Kraus operators of size {int(np.sqrt(S.shape[0]))} do not match {len(ws)} wire(s)")
         if len(ws) > 5:
             raise ValueError("channels act on at most 5 wires (a 2^(2k) superoperator, 2k <= 10)")
-        mat = torch.tensor(S, dtype=C_DTYPE, device=self.reg._sv_device())
+        mat = torch.from_numpy(S.astype(np.complex64))
         reg_wires = tuple(ws) + tuple(w + n for w in ws)
         self.reg._push(E.TapeOp("qubitunitaryfast", reg_wires, mat, False, mat._version, nonunitary=True))
 
-    def amplitude_damping(self, wires, gamma: float):
+    def _each(self, wires, kraus_ops: Sequence[np.ndarray]):
+        S = superoperator(kraus_ops)
         for w in ([wires] if isinstance(wires, (int, np.integer)) else wires):
-            self.kraus(int(w), amplitude_damping_kraus(gamma))
+            self._channel(int(w), S)
+
+    def amplitude_damping(self, wires, gamma: float):
+        self._each(wires, amplitude_damping_kraus(gamma))
 
     def phase_damping(self, wires, lam: float):
-        for w in ([wires] if isinstance(wires, (int, np.integer)) else wires):
-            self.kraus(int(w), phase_damping_kraus(lam))
+        self._each(wires, phase_damping_kraus(lam))
 
     def depolarizing(self, wires, p: float):
-        for w in ([wires] if isinstance(wires, (int, np.integer)) else wires):
-            self.kraus(int(w), depolarizing_kraus(p))
+        self._each(wires, depolarizing_kraus(p))
 
     def bit_flip(self, wires, p: float):
-        for w in ([wires] if isinstance(wires, (int, np.integer)) else wires):
-            self.kraus(int(w), bit_flip_kraus(p))
+        self._each(wires, bit_flip_kraus(p))
 
     def phase_flip(self, wires, p: float):
-        for w in ([wires] if isinstance(wires, (int, np.integer)) else wires):
-            self.kraus(int(w), phase_flip_kraus(p))
+        self._each(wires, phase_flip_kraus(p))
 
     # ------------------------------------------------------------ state
     @property
@@ -226,20 +232,25 @@ class NoiseDevice(nn.Module):
 # ----------------------------------------------------------------------------
 # expectations on densities: Tr(rho P) for Pauli strings
 # ----------------------------------------------------------------------------
-def _pauli_masks(obs: str):
-    n = len(obs)
-    x = z = ny = 0
-    for w, ch in enumerate(obs.upper()):
-        bit = 1 << (n - 1 - w)
-        if ch in "XY":
-            x |= bit
-        if ch in "ZY":
-            z |= bit
-        if ch == "Y":
-            ny += 1
-        if ch not in "IXYZ":
-            raise ValueError(f"unknown Pauli character '{ch}' in '{obs}'")
-    return x, z, ny
+def _string_tables(n: int, observables: Sequence[str]):
+    """For T strings: the gathered index r * 2^n + (r ^ x) and its sign
+    (-1)^popcount(r & z), [T, 2^n] each, and i^nY as its real and imaginary
+    parts, [T] each."""
+    d = 1 << n
+    masks = [pauli_masks(obs, n) for obs in observables]
+    x, z, ny = (np.array(v, dtype=np.int64) for v in zip(*masks))
+    r = np.arange(d, dtype=np.int64)
+    par = r & z[:, None]
+    for sh in (16, 8, 4, 2, 1):
+        par ^= par >> sh
+    ph = _PHASE[ny % 4]
+    return (r * d + (r ^ x[:, None]), (1 - 2 * (par & 1)).astype(np.float32),
+            ph.real.astype(np.float32), ph.imag.astype(np.float32))
+
+
+_small_tables = functools.lru_cache(maxsize=32)(_string_tables)
+SMALL_TABLE = 1 << 16          # entries of a table that is kept for the next call with the same strings
+CHUNK = 1 << 22                # entries gathered per row at a time
 
 
 def density_expval_strings(dev: NoiseDevice, observables: Sequence[str]) -> torch.Tensor:
@@ -247,21 +258,17 @@ def density_expval_strings(dev: NoiseDevice, observables: Sequence[str]) -> torc
 
     P|r> = i^{nY} (-1)^{popcount(r & z)} |r ^ x>, so
     Tr(rho P) = i^{nY} sum_r (-1)^{popcount(r & z)} rho[r, r ^ x]:
-    a gather of 2^n entries of the 4^n per row (differentiable; the gradient
-    reaches the gates through the engine's adjoint sweep)."""
+    a gather of 2^n entries of the 4^n per row and string (differentiable; the
+    gradient reaches the gates through the engine's adjoint sweep)."""
     n = dev.n_wires
     flat = dev.reg.get_states_1d()                         # [bsz, 4^n]
     d = 1 << n
-    r = np.arange(d, dtype=np.int64)
     cols = []
-    for obs in observables:
-        if len(obs) != n:
-            raise ValueError(f"observable '{obs}' has {len(obs)} characters for {n} wires")
-        x, z, ny = _pauli_masks(obs)
-        idx = torch.from_numpy(r * d + (r ^ x)).to(flat.device)
-        par = np.array([bin(v).count("1") & 1 for v in (r & z)], dtype=np.float32) if z else np.zeros(d, np.float32)
-        sgn = torch.from_numpy(1.0 - 2.0 * par).to(flat.device)
-        s = (flat[:, idx] * sgn).sum(-1)                       # sum_r sign rho[r, r^x]
-        ph = 1j ** ny                                          # Re(i^ny s)
-        cols.append(s.real * ph.real - s.imag * ph.imag)
-    return torch.stack(cols, dim=-1)
+    per = max(1, CHUNK >> n)
+    for t0 in range(0, len(observables), per):
+        obs = tuple(observables[t0:t0 + per])
+        idx, sgn, re, im = (_small_tables if len(obs) * d <= SMALL_TABLE else _string_tables)(n, obs)
+        g = flat[:, E.upload(idx.reshape(-1), flat.device)].reshape(-1, len(obs), d)
+        s = (g * E.upload(sgn, flat.device)).sum(-1)           # sum_r sign rho[r, r^x]
+        cols.append(s.real * E.upload(re, flat.device) - s.imag * E.upload(im, flat.device))    # Re(i^ny s)
+    return torch.cat(cols, dim=-1)

@@ -12,6 +12,7 @@ import numpy as np
 import torch
 import torch.nn as nn
 
+from .. import _native as N
 from .. import functional as tqf
 from .. import gates as G
 from ..macro import C_DTYPE, F_DTYPE
@@ -118,6 +119,36 @@ class Operator(QuantumModule):
 
     def __repr__(self):
         return f" class: {self.name} \n parameters: {self.params} \n wires: {self.wires} \n inverse: {self.inverse}"
+
+
+def apply_each(q_device, ops, wires):
+    """``op(q_device, wires=w)`` for each op and its wires, in order.  Ops of
+    this module's classes that nothing intercepts (no hooks, no tracing, no
+    replaced forward, no op history) are recorded without the module call."""
+    n = q_device.n_wires
+    plain = not (getattr(q_device, "record_op", False) or torch._C._get_tracing_state()
+                 or torch.nn.modules.module._has_any_global_hook())
+    specs = {}
+    for op, w in zip(ops, wires):
+        if plain:
+            cls = type(op)
+            spec = specs.get(cls)
+            if spec is None:
+                spec = specs[cls] = _plain_spec(cls)
+            if spec:
+                t = N.host().operator_op(op, spec, w, n)
+                if t is not None:
+                    q_device._push(t)
+                    continue
+        op(q_device, wires=w)
+
+
+def _plain_spec(cls):
+    """(gate, wires, parameters) of a class whose call only records that gate, else ()."""
+    if not issubclass(cls, Operator) or cls.forward is not Operator.forward or cls.__call__ is not nn.Module.__call__ \
+            or cls.__getattr__ is not nn.Module.__getattr__ or cls.__setattr__ is not nn.Module.__setattr__:
+        return ()
+    return getattr(cls.func, "plain_spec", None) or ()
 
 
 class Observable(Operator, metaclass=ABCMeta):
