@@ -511,3 +511,91 @@ def test_dense_kq_lds_staged(k, batched):
         ref = np.stack([_dense_apply_np(init[b:b + 1], mats[b if batched else 0], bits, cmask, cval, n)[0]
                         for b in range(bsz)])
         assert np.abs(st.cpu().numpy() - ref).max() < 1e-5, (k, batched, n, bsz, nctrl)
+
+
+def _pauli_apply_ref(psi, n, obs):
+    """P psi in float64 ([bsz, 2^n] complex128)."""
+    x = sum(1 << (n - 1 - w) for w, c in enumerate(obs) if c in "XY")
+    z = sum(1 << (n - 1 - w) for w, c in enumerate(obs) if c in "ZY")
+    src = np.arange(1 << n) ^ x
+    par = np.array([bin(v & z).count("1") & 1 for v in range(1 << n)])[src]
+    return psi[:, src] * np.where(par, -1.0, 1.0) * 1j ** obs.count("Y")
+
+
+@gpu
+@pytest.mark.parametrize("n,bsz,terms", [(8, 3, 5), (9, 1, 40), (12, 3, 97), (13, 2, 130), (14, 1, 33), (16, 3, 20),
+                                         (13, 1, 17), (10, 2, 200)])
+def test_pauli_sets_of_every_width(n, bsz, terms):
+    """Values and state gradients of many strings at once: every set width, more terms than a set holds, entries
+    of one and of many terms, strings that flip more bits than a set has room for, diagonal strings alone.
+    Amplitudes of size 2^(-n/2) in float32 sum to an expectation with an error near 2^-23; 1e-5 is allowed as
+    everywhere here, and for the gradient 1e-5 of the largest possible entry, 2 sum |c|."""
+    import torchquantum_amd as tq
+    rng = np.random.default_rng(100 * n + terms)
+    psi = rng.normal(size=(bsz, 1 << n)) + 1j * rng.normal(size=(bsz, 1 << n))
+    psi /= np.linalg.norm(psi, axis=1, keepdims=True)
+    obs = set()
+    while len(obs) < min(terms, 3 ** n):
+        k = int(rng.integers(1, n + 1)) if rng.random() < 0.2 else int(rng.integers(1, 4))
+        o = ["I"] * n
+        letters = "Z" if terms == 17 or rng.random() < 0.3 else "XYZ"
+        for w in rng.choice(n, k, replace=False):
+            o[w] = str(rng.choice(list(letters)))
+        obs.add("".join(o))
+    obs = sorted(obs)
+    c = rng.uniform(-1, 1, len(obs))
+    psi = psi.astype(np.complex64).astype(np.complex128)
+    P = [_pauli_apply_ref(psi, n, o) for o in obs]
+    values = np.stack([(psi.conj() * p).sum(1).real for p in P], 1)
+    st = torch.tensor(psi, dtype=torch.complex64, device="cuda", requires_grad=True)
+    q = tq.QuantumDevice(n_wires=n, bsz=bsz, device="cuda")
+    q.set_states(st)
+    got = tq.expval_joint_analytical_batch(q, obs)
+    assert np.abs(got.detach().cpu().numpy() - values).max() < 1e-5
+    g = torch.tensor(rng.uniform(0.5, 2, (bsz, len(obs))), dtype=torch.float32, device="cuda")
+    (grad,) = torch.autograd.grad((got * g).sum(), st)
+    gn = g.cpu().numpy().astype(np.float64)
+    want = sum(2 * gn[:, t:t + 1] * P[t] for t in range(len(obs)))
+    assert np.abs(grad.cpu().numpy() - want).max() < 1e-5 * 2 * gn.sum(1).max()
+    total = tq.expval_pauli_sum(q, obs, c)
+    assert np.abs(total.detach().cpu().numpy() - values @ c).max() < 1e-5 * max(1.0, np.abs(c).sum())
+    (grad,) = torch.autograd.grad(total.sum(), st)
+    want = sum(2 * c[t] * P[t] for t in range(len(obs)))
+    assert np.abs(grad.cpu().numpy() - want).max() < 1e-5 * 2 * np.abs(c).sum()
+
+
+@gpu
+def test_pauli_sets_at_the_highest_positions():
+    """29 wires: sets whose local positions are beyond what buffer instructions reach.  A product state of RY, RX
+    angles, so that a string's value is the product of its wires' own: <X> = sin t and <Z> = cos t under RY(t),
+    <Y> = -sin t under RX(t), and derivatives follow."""
+    import torchquantum_amd as tq
+    n = 29
+    t = torch.linspace(0.3, 1.7, n, dtype=torch.float64)
+    p = [t[w].to(torch.float32).reshape(1, 1).cuda().requires_grad_() for w in range(n)]
+    q = tq.QuantumDevice(n_wires=n, bsz=1, device="cuda")
+    for w in range(n):
+        (tq.functional.rx if w % 3 == 2 else tq.functional.ry)(q, w, params=p[w])
+
+    def term(d):
+        return "".join(d.get(w, "I") for w in range(n))
+
+    def val(d, tt):
+        v = 1.0
+        for w, c in d.items():
+            v = v * {("X", 0): torch.sin(tt[w]), ("Z", 0): torch.cos(tt[w]), ("Z", 1): torch.cos(tt[w]),
+                     ("Y", 1): -torch.sin(tt[w])}[(c, int(w % 3 == 2))]
+        return v
+
+    ds = [{0: "X", 1: "X"}, {0: "X", 28: "Z"}, {2: "Y", 5: "Y"}, {0: "Z", 2: "Z"}, {3: "X", 2: "Y", 27: "X"},
+          {4: "X", 0: "Z"}, {6: "X"}, {7: "X"}, {9: "X", 10: "X"}, {12: "X", 13: "X", 14: "Y"}, {1: "Z"}]
+    got = tq.expval_joint_analytical_batch(q, [term(d) for d in ds])[0].detach().cpu().double()
+    assert (got - torch.stack([val(d, t) for d in ds])).abs().max() < 1e-5
+    tr = t.clone().requires_grad_()
+    c = [0.5 + 0.1 * i for i in range(len(ds))]
+    want = sum(k * val(d, tr) for k, d in zip(c, ds))
+    (wg,) = torch.autograd.grad(want, tr)
+    total = tq.expval_pauli_sum(q, [term(d) for d in ds], c).sum()
+    assert abs(float(total.detach()) - float(want.detach())) < 1e-5 * sum(c)
+    grads = torch.cat([x.reshape(-1) for x in torch.autograd.grad(total, p)]).cpu().double()
+    assert (grads - wg).abs().max() < 1e-5 * sum(c)
