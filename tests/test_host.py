@@ -736,3 +736,38 @@ def test_default_stage_width_follows_state_size():
     assert E.choose_stage_bits(20, o, 16) == 12          # 128 MiB
     assert E.choose_stage_bits(10, o, 1 << 20) == 10     # many rows, few qubits
     assert E.choose_stage_bits(24, E.EngineOptions(stage_bits=11), 64) == 11
+
+
+@pytest.mark.parametrize("n,stage_bits,io", [(6, 4, True), (7, 6, False), (11, 10, True), (5, 5, True)])
+def test_swaps_move_no_data_inside_a_stage(n, stage_bits, io):
+    """Uncontrolled SWAPs inside a stage rename local bits: no dense op for them, the same state (also from a given
+    one, un-computed by the adjoint) and the same gradients, with the input layer pruned where the wires that a
+    SWAP brought together allow it.  Tolerances as in the tests above (complex64 matrices)."""
+    rng = np.random.default_rng(1700 + n)
+    bsz = 2
+    names = ["swap", "swap", "swap", "rx", "u3", "cnot", "cz", "rz", "toffoli", "crx"]
+    ops = [dict(name="ry", wires=[w], params=rng.uniform(0, np.pi, size=(bsz, 1)), inverse=False) for w in range(n)]
+    train = random_ops(n, 60, bsz, rng, names=names)
+    tape = _tape_from_ops(ops) + _tape_from_ops(train, grad=True)
+    ops = ops + train
+    c = E.Compiled(tape, n, bsz, E.EngineOptions(stage_bits=stage_bits, io_layouts=io), "cpu")
+    stages = [p[1] for kind, p in c.steps if kind == "stage"]
+    assert any(st.moved for st in stages)
+    for st in stages:
+        assert not int(st.words[E.H_FLAGS]) & E.FEAT_MAT2
+        assert sorted(st.moved) == sorted(st.moved.values())
+    pool = c.pool_host(tape, True, True).astype(np.complex128)
+    init = rng.normal(size=(bsz, 2 ** n)) + 1j * rng.normal(size=(bsz, 2 ** n))
+    psi = EM.run_compiled(c, pool, init)
+    assert np.abs(psi - O.run_ops(oracle_ops(ops, bsz), n, bsz, state=init)).max() < 5e-6
+    cvec = rng.normal(size=(bsz, 2 ** n)) + 1j * rng.normal(size=(bsz, 2 ** n))
+    back, lam = psi.copy(), cvec.copy()
+    full = EM.adjoint_compiled(c, pool, back, lam)
+    assert np.abs(back - init).max() < 1e-5
+    assert np.abs(O.run_ops(oracle_ops(ops, bsz), n, bsz, state=lam) - cvec).max() < 1e-5
+    pruned = EM.adjoint_compiled(c, pool, psi.copy(), cvec.copy(), need_input_grad=False)
+    assert np.abs(pruned - full).max() < 1e-6 * (1 + np.abs(full).max())
+    want = EM.adjoint_compiled(E.Compiled(tape, n, bsz, E.EngineOptions(mode="pergate", adjoint_mg=False), "cpu"),
+                               E.Compiled(tape, n, bsz, E.EngineOptions(mode="pergate", adjoint_mg=False), "cpu")
+                               .pool_host(tape, True, True).astype(np.complex128), psi.copy(), cvec.copy())
+    assert np.abs(full[:, :c.n_slots] - want[:, :c.n_slots]).max() < 1e-5 * (1 + np.abs(want).max())
