@@ -57,9 +57,9 @@ class CircuitBatch:
         """circuits: [(n_wires, ops)], ops as {name, wires, params, inverse} dicts.
         options: per-circuit EngineOptions (mode is forced to 'fused').
         mode: "queue" (one persistent launch) or "levels" (a launch per level).
-        groups_per_item: groups of 2^m amplitudes per work item (default 8
-        with the queue, 4 with a launch per level: the measured best of
-        2..32 on the 256-circuit workload, 21.6 and 24.8 ms)."""
+        groups_per_item: groups of 2^m amplitudes per work item.  Default
+        with the queue: see _groups_per_item; with a launch per level 4 (the
+        measured best of 2..32 on the 256-circuit workload, 24.8 ms)."""
         lib = N.lib()
         if (lib.tqsv_batch_item_bytes() != BATCH_ITEM.itemsize or lib.tqsv_batch_zcirc_bytes() != ZCIRC.itemsize
                 or lib.tqsv_batch_queue_item_bytes() != QUEUE_ITEM.itemsize):
@@ -67,9 +67,9 @@ class CircuitBatch:
         if mode not in ("queue", "levels"):
             raise ValueError(f"unknown batch mode {mode!r}")
         self.mode = mode
-        if groups_per_item is None:
-            groups_per_item = 8 if mode == "queue" else 4
-        if groups_per_item < 1:
+        if groups_per_item is None and mode == "levels":
+            groups_per_item = 4
+        if groups_per_item is not None and groups_per_item < 1:
             raise ValueError("groups_per_item must be positive")
         self.device = torch.device(device)
         self.n_circ = len(circuits)
@@ -122,6 +122,7 @@ class CircuitBatch:
         self.mats = torch.from_numpy(np.concatenate(pools).astype(np.complex64)).to(self.device)
         # work lists per level, and the same items as one level-major queue
         n_levels = max(len(o) for o in self.stage_offsets)
+        per_item = [groups_per_item] * self.n_circ if groups_per_item is not None else self._groups_per_item()
         self.levels = []
         queue = []
         seen = [0] * self.n_circ          # items of each circuit in earlier levels
@@ -133,9 +134,9 @@ class CircuitBatch:
                     continue
                 m = self.stage_m[i][L]
                 ng = 1 << (self.ns[i] - m)
-                for g0 in range(0, ng, groups_per_item):
+                for g0 in range(0, ng, per_item[i]):
                     b = (self.state_off[i], self.stage_offsets[i][L], self.ns[i], 1 if L == 0 else 0, 0,
-                         g0, min(g0 + groups_per_item, ng))
+                         g0, min(g0 + per_item[i], ng))
                     items.append(b)
                     queue.append((b, i, seen[i]))
                     per_circ[i] += 1
@@ -164,6 +165,21 @@ class CircuitBatch:
         self.part = torch.empty(self.n_chunks, dtype=torch.float32, device=self.device)
         self.out = torch.empty(self.n_circ, dtype=torch.float32, device=self.device)
         self.graph = None
+
+    def _groups_per_item(self) -> List[int]:
+        """Groups per work item of each circuit.  Few per item leave a level
+        more items than the 1024 resident workgroups; many leave workgroups
+        idle, and the deepest circuit's stages, each waiting for the one
+        before, one after another on few of them.  So: as many groups as give
+        a mean level about 1536 items, at most 6 (a claim of an item costs
+        about 50 ns on one counter), and at least 4 items per stage.  Measured, 1 / 2 / 4 / 8 groups for all: 64 circuits of
+        up to 22 qubits 11.5 / 6.8 / 6.0 / 7.1 ms, 256 of them 34.9 / 20.1 /
+        17.0 / 17.1 ms, 20 of up to 20 qubits 1.17 / 1.10 / 1.64 / 3.0 ms, 30
+        of up to 14 qubits 0.31 / 0.53 / 0.98 / 0.97 ms."""
+        groups = [[1 << (n - m) for m in ms] for n, ms in zip(self.ns, self.stage_m)]
+        mean = sum(map(sum, groups)) / max(map(len, groups))
+        most = max(1, min(6, round(mean / 1536)))
+        return [max(1, min(most, max(g) // 4)) for g in groups]
 
     @property
     def n_launches(self) -> int:

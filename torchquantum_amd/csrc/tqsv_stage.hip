@@ -844,7 +844,32 @@ struct BatchItem {
   int64_t g0, g1;      // group range of this item
 };
 
+// State accesses of the queue kernel: relaxed agent-scope atomics of 8 bytes,
+// which go past the XCDs' separate L2 caches, so that one XCD's finished stores
+// are what another loads.  With plain accesses every item ended with an L2
+// write-back and every wait with an invalidation, which the other workgroups
+// of the XCD paid for too (64 circuits: 7.46 -> 7.14 ms).
+template <bool COHERENT>
+__device__ __forceinline__ float2 state_load(const float2* p) {
+  if constexpr (COHERENT) {
+    const uint64_t v = __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+  } else {
+    return *p;
+  }
+}
+template <bool COHERENT>
+__device__ __forceinline__ void state_store(float2* p, float2 v) {
+  if constexpr (COHERENT) {
+    const uint64_t b = (uint64_t)__float_as_uint(v.x) | (uint64_t)__float_as_uint(v.y) << 32;
+    __hip_atomic_store((uint64_t*)p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    *p = v;
+  }
+}
+
 // One item: a stage program over groups [g0, g1) of one circuit's state.
+template <bool COHERENT>
 __device__ __forceinline__ void batch_item(float2* __restrict__ states, const BatchItem& item,
                                            const int* __restrict__ progs, const float2* __restrict__ mats,
                                            float2* lds, int tid) {
@@ -869,7 +894,7 @@ __device__ __forceinline__ void batch_item(float2* __restrict__ states, const Ba
     } else if (active) {
       const float2* src = st + (uint64_t)goff + toff;
 #pragma unroll
-      for (int j = 0; j < NS; ++j) a[j] = src[roff[j]];
+      for (int j = 0; j < NS; ++j) a[j] = state_load<COHERENT>(src + roff[j]);
     }
     for (int o = 0; o < n_ops; ++o) {
       const int* __restrict__ w = ops + 8 * o;
@@ -884,7 +909,7 @@ __device__ __forceinline__ void batch_item(float2* __restrict__ states, const Ba
       float2* dst = st + (uint64_t)goff + soff;
       asm volatile("" : "+v"(dst));
 #pragma unroll
-      for (int j = 0; j < NS; ++j) dst[sroff[j]] = a[j];
+      for (int j = 0; j < NS; ++j) state_store<COHERENT>(dst + sroff[j], a[j]);
     }
   }
 }
@@ -895,7 +920,7 @@ __global__ __launch_bounds__(BATCH_THREADS) void k_batch_fwd(float2* __restrict_
                                                              const float2* __restrict__ mats) {
   extern __shared__ float2 lds[];
   for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
-    batch_item(states, items[it], progs, mats, lds, threadIdx.x);
+    batch_item<false>(states, items[it], progs, mats, lds, threadIdx.x);
     __syncthreads();
   }
 }
@@ -906,9 +931,8 @@ __global__ __launch_bounds__(BATCH_THREADS) void k_batch_fwd(float2* __restrict_
 // order from a global counter (ctrl[0]), so whenever a workgroup waits, every
 // item it waits for is already held by a running workgroup, and the earliest
 // unfinished item never waits: the queue drains with any grid size.  A
-// finished item is published with a device-scope release (its stores, then
-// done[c] += 1); a waiting workgroup polls done[c] with acquire loads, at
-// most spin_limit times: past that it sets ctrl[1] (the results are then
+// finished item is published by done[c] += 1 once its stores are in memory; a
+// waiting workgroup polls done[c], at most spin_limit times: past that it sets ctrl[1] (the results are then
 // wrong and the host reports it) and goes on, as does every later wait once
 // ctrl[1] is set, so every wave reaches the queue's end.
 struct QueueItem {
@@ -930,12 +954,11 @@ __global__ void k_queue_reset(int* __restrict__ ctrl, int* __restrict__ done, in
 // of the loop that the other lanes keep running -- past their barrier -- so
 // the loop never ends.)  Only wave 0 claims, waits and publishes:
 //   claim    one atomic add on the queue counter;
-//   wait     relaxed polls of done[c], then one device-scope acquire fence
-//            (it invalidates this CU's L1 and this XCD's L2, which the
-//            workgroup's other waves, ordered after it by the barrier, share);
-//   publish  every wave waits for its stores (workgroup-scope release), the
-//            barrier, then wave 0's device-scope release (L2 write-back) and
-//            a relaxed add to done[c].
+//   wait     relaxed polls of done[c]; the workgroup's loads of the state come
+//            after the barrier that follows, and go past L1 and L2
+//            (state_load);
+//   publish  every wave waits until its stores, which go past L2 too, have
+//            reached memory, the barrier, then wave 0's relaxed add to done[c].
 __global__ __launch_bounds__(BATCH_THREADS) void k_batch_queue(float2* __restrict__ states,
                                                                const QueueItem* __restrict__ items, int n_items,
                                                                const int* __restrict__ progs,
@@ -972,14 +995,12 @@ __global__ __launch_bounds__(BATCH_THREADS) void k_batch_queue(float2* __restric
           break;
         __builtin_amdgcn_s_sleep(8);
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();                           // the wait is over, the previous item's LDS use too
-    batch_item(states, q.b, progs, mats, lds, tid);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");   // this wave's stores are done
+    batch_item<true>(states, q.b, progs, mats, lds, tid);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's stores have reached memory
     __syncthreads();                           // ... in every wave; s_item has been read
     if (wave0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       __hip_atomic_fetch_add(&done[q.circ], one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
