@@ -46,6 +46,14 @@ KERNELS_PER_SOURCE = 4
 # to 160-190 VGPRs.  Measured on the 24-qubit gradient: 531 -> 500 ms.  The
 # forward kernels gain nothing from it.
 COMPILE_OPTS = {"f": "", "a": "-mllvm -amdgpu-sched-strategy=iterative-maxocc"}
+# Forward kernels are held to four waves per SIMD, i.e. at most 128 VGPRs.
+# Their LDS lets that many run (two 512-thread workgroups per CU with 13
+# local bits, four 256-thread ones with 12), but LLVM takes 130-140 VGPRs for
+# some 13-bit stages, which leaves one workgroup per CU and nothing to run
+# while it waits at a remap barrier.  Measured over the 30-qubit bsz-4 layer
+# circuit (35 stages): 632.7 -> 583.3 ms.  12-bit stages stay below 128 by themselves
+# (20 qubits bsz 16: unchanged).
+FWD_WAVES_PER_EU = 4
 COMPILE_OPTS["p"] = COMPILE_OPTS["a"]     # pruned adjoint stages (gen_adjoint with skip / no_store)
 # Code-generation defaults (gen_forward / gen_adjoint arguments of the same
 # names), chosen by timing the stages of the 24-qubit bsz-64 gradient on
@@ -1003,7 +1011,8 @@ def gen_forward(words: np.ndarray, name: str, nontemporal: bool = False, buf: Op
     body = ["  " + s for s in g.lines]
     stores = [f"      {_store(sp, 'out', j, a[j], mode, lay='st')}" for j in range(NS)]
     nt = 1 << sp.T
-    src = [f'extern "C" __global__ void __launch_bounds__({nt}) {name}(float2* __restrict__ out, '
+    src = [f'extern "C" __global__ void __launch_bounds__({nt}) '
+           f'__attribute__((amdgpu_waves_per_eu({FWD_WAVES_PER_EU}))) {name}(float2* __restrict__ out, '
            "const float2* __restrict__ in, const float2* __restrict__ mats, int init_zero, long long n_groups, "
            "long long gpw) {"]
     if g.used_lds:
@@ -1209,6 +1218,8 @@ def kernel_name(kind: str, prog, nt: bool = False) -> str:
     if extra:
         hs.update(repr(sorted(extra.items())).encode())
     hs.update(COMPILE_OPTS[kind].encode())
+    if kind == "f":
+        hs.update(f"w{FWD_WAVES_PER_EU}".encode())
     hs.update(repr((_codegen(None, None, kind), _mfma(kind), _lane(kind))).encode())
     if nt:
         hs.update(b"nt")
