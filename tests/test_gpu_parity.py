@@ -599,3 +599,26 @@ def test_pauli_sets_at_the_highest_positions():
     assert abs(float(total.detach()) - float(want.detach())) < 1e-5 * sum(c)
     grads = torch.cat([x.reshape(-1) for x in torch.autograd.grad(total, p)]).cpu().double()
     assert (grads - wg).abs().max() < 1e-5 * sum(c)
+
+
+@gpu
+@pytest.mark.parametrize("stage_bits", [5, 7, 8, 10, 12])
+def test_remaps_of_every_thread_count(stage_bits):
+    """Stages of 2 to 256 threads with many register remaps, forward and
+    adjoint.  States within 1e-5 of the oracle; gradients within 5e-5 of the
+    per-gate kernels' (unit states, observables of norm <= 26, about 100
+    operations of rounding 6e-8 each whose errors add as a random walk)."""
+    import torchquantum_amd as tq
+    n, bsz = 13, 3
+    rng = np.random.default_rng(70 + stage_bits)
+    ops = random_ops(n, 90, bsz, rng, names=["rx", "u3", "cnot", "cz", "rzz", "crx", "swap", "rxx", "toffoli"])
+    assert np.abs(_run(n, bsz, ops, "fused", stage_bits=stage_bits)
+                  - O.run_ops(oracle_ops(ops, bsz), n, bsz)).max() < 1e-5
+    obs, coef = config3_observables(n)
+    grads = []
+    for mode, kw in (("fused", {"stage_bits": stage_bits}), ("pergate", {})):
+        q = _qdev(n, bsz, mode, **kw)
+        ts = apply_ops_tq(q, ops, DEV, requires_grad=True)
+        tq.expval_pauli_sum(q, obs, coef).sum().backward()
+        grads.append(torch.cat([t.grad.reshape(-1) for t in ts]).cpu())
+    assert (grads[0] - grads[1]).abs().max() < 5e-5

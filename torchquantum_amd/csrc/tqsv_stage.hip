@@ -364,8 +364,7 @@ __device__ __forceinline__ void f_xperm(float2 (&a)[NS], bool tok, int rm, int r
   for (int j = 0; j < NS; ++j) {
     if (j & (1 << K)) continue;
     const int j1 = j | (1 << K);
-    if ((j & rm) != rv) continue;  // register controls: a wave-uniform skip
-    const bool ok = tok;
+    const bool ok = tok & ((j & rm) == rv);
     const float2 x0 = a[j], x1 = a[j1];
     a[j] = csel(ok, x1, x0);
     a[j1] = csel(ok, x0, x1);
@@ -374,49 +373,78 @@ __device__ __forceinline__ void f_xperm(float2 (&a)[NS], bool tok, int rm, int r
 
 // sign flip where the controls match (Z, CZ, CCZ): phase -1, no parity
 __device__ __forceinline__ void f_sign(float2 (&a)[NS], bool tok, int rm, int rv) {
+  const int flip = tok ? (int)0x80000000 : 0;
 #pragma unroll
   for (int j = 0; j < NS; ++j) {
-    if ((j & rm) != rv) continue;  // register controls: a wave-uniform skip
-    const bool ok = tok;
-    a[j] = make_float2(ok ? -a[j].x : a[j].x, ok ? -a[j].y : a[j].y);
+    const int f = (j & rm) == rv ? flip : 0;
+    a[j].x = __int_as_float(__float_as_int(a[j].x) ^ f);
+    a[j].y = __int_as_float(__float_as_int(a[j].y) ^ f);
   }
 }
 
 // ------------------------------------------------------------------ remap
-__device__ __forceinline__ int layout_thread(const int* __restrict__ tl, int T, int tid) {
-  int lt = 0;
-  for (int i = 0; i < T; ++i) lt |= ((tid >> i) & 1) ? tl[i] : 0;
-  return lt;
+// Bound, on states that leave a few wavefronts per SIMD, by the latency of
+// scalar loads: walking a record bit by bit cost one of them per thread bit
+// and layout, each waited for in turn.  All words of a record now come in
+// independent loads at fixed places, an op's words in one (op_words), and
+// adjoint remaps read a record once for psi and lam.  Stage launches: 10
+// qubits bsz 256 (95 ops, 15 remaps) forward 87 -> 70 us, adjoint 151 -> 105;
+// 13 qubits bsz 37 25.2 -> 21.7 and 43.8 -> 33.0; 20 wires bsz 3 35.6 -> 31.6;
+// 64 circuits in one queue launch 5.96 -> 5.27 ms.
+//
+// A layout record holds the local-index value of each thread bit, tl[T], and
+// of each register bit, rl[R].  swz is linear over XOR, so a slot's LDS index
+// is swz(thread part) ^ swz(slot part), the slot part being wave-uniform.
+struct Layout {
+  int t;        // byte offset of this thread's slot 0
+  int r[R];     // what register bit k toggles in it
+};
+
+constexpr int T_MAX = 9;   // m <= 13
+
+// The layout of the record that ends at `end`.  The T_MAX + R words before
+// `end` are read whatever T is, so that they are independent loads at fixed
+// places (two or three wide ones): a record shorter than that is preceded by
+// the stage's header, ops and other records, and the words before it meet
+// the zero low bits of stid = tid << (T_MAX - T).
+__device__ __forceinline__ Layout layout_ending(const int* __restrict__ end, int stid) {
+  const int* __restrict__ w = end - (T_MAX + R);
+  int t = 0;
+#pragma unroll
+  for (int i = 0; i < T_MAX; ++i) t ^= w[i] & -((stid >> i) & 1);
+  Layout L;
+  L.t = swz(t) << 3;
+#pragma unroll
+  for (int k = 0; k < R; ++k) L.r[k] = swz(w[T_MAX + k]) << 3;
+  return L;
 }
 
-__device__ __forceinline__ void remap(float2 (&a)[NS], float2* __restrict__ lds, const int* __restrict__ from,
-                                      const int* __restrict__ to, int T, int tid, bool active = true) {
-  // record: tl[T], rl[R] (local-index value of each thread / register bit).
-  // swz is linear over XOR, so address = swz(thread part) ^ swz(slot part),
-  // the slot part being wave-uniform.
-  int st0 = swz(layout_thread(from, T, tid));
+// Slots in Gray-code order: each address is the one before with one register
+// bit's offset toggled.
+__device__ __forceinline__ void lds_put(const float2 (&a)[NS], float2* __restrict__ lds, const Layout& L) {
+  int at = L.t;
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    if (i > 0) at ^= L.r[__builtin_ctz(i)];
+    *(float2*)((char*)lds + at) = a[i ^ (i >> 1)];
+  }
+}
+
+__device__ __forceinline__ void lds_get(float2 (&a)[NS], const float2* __restrict__ lds, const Layout& L) {
+  int at = L.t;
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    if (i > 0) at ^= L.r[__builtin_ctz(i)];
+    a[i ^ (i >> 1)] = *(const float2*)((const char*)lds + at);
+  }
+}
+
+__device__ __forceinline__ void remap(float2 (&a)[NS], float2* __restrict__ lds, const Layout& from,
+                                      const Layout& to, bool active = true) {
   __syncthreads();
-  if (active) {
-#pragma unroll
-  for (int j = 0; j < NS; ++j) {
-    int lr = 0;
-#pragma unroll
-    for (int k = 0; k < R; ++k) lr |= ((j >> k) & 1) ? from[T + k] : 0;
-    asm volatile("" : "+v"(st0));
-    lds[st0 ^ swz(lr)] = a[j];
-  }
-  }
+  if (active) lds_put(a, lds, from);
   __syncthreads();
-  if (!active) return;
-  int st1 = swz(layout_thread(to, T, tid));
-#pragma unroll
-  for (int j = 0; j < NS; ++j) {
-    int lr = 0;
-#pragma unroll
-    for (int k = 0; k < R; ++k) lr |= ((j >> k) & 1) ? to[T + k] : 0;
-    asm volatile("" : "+v"(st1));
-    a[j] = lds[st1 ^ swz(lr)];
-  }
+  if (active) lds_get(a, lds, to);
 }
 
 // ------------------------------------------------------------------ dispatch
@@ -424,8 +452,22 @@ __device__ __forceinline__ void remap(float2 (&a)[NS], float2* __restrict__ lds,
 // Stages without them run a leaner instantiation (fewer live registers).
 constexpr int FEAT_MAT2 = 1, FEAT_MATK = 2;
 
+// One op's words, fetched together (and at once) by scalar loads.
+struct OpWords {
+  int v[8];
+  __device__ __forceinline__ int operator[](int i) const { return v[i]; }
+};
+
+__device__ __forceinline__ OpWords op_words(const int* __restrict__ p) {
+  OpWords w;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w.v[i] = p[i];
+  asm volatile("" : "+s"(w.v[0]), "+s"(w.v[1]), "+s"(w.v[2]), "+s"(w.v[3]), "+s"(w.v[4]), "+s"(w.v[5]), "+s"(w.v[6]), "+s"(w.v[7]));
+  return w;
+}
+
 template <int FEAT>
-__device__ __forceinline__ void fwd_op(float2 (&a)[NS], const int* __restrict__ w, const float2* __restrict__ M,
+__device__ __forceinline__ void fwd_op(float2 (&a)[NS], const OpWords& w, const float2* __restrict__ M,
                                        int tid) {
   const int type = w[0] & 15;
   const int fl = w[0];
@@ -498,7 +540,7 @@ __device__ __forceinline__ void fwd_op(float2 (&a)[NS], const int* __restrict__ 
 }
 
 template <int FEAT>
-__device__ __forceinline__ void bwd_op(float2 (&p)[NS], float2 (&l)[NS], const int* __restrict__ w,
+__device__ __forceinline__ void bwd_op(float2 (&p)[NS], float2 (&l)[NS], const OpWords& w,
                                        const float2* __restrict__ M, int tid, float (&g8)[8]) {
   float (&g)[4] = *reinterpret_cast<float (*)[4]>(&g8[0]);
   const int type = w[0] & 15;
@@ -604,17 +646,27 @@ __device__ __forceinline__ void layout_offsets(const int* __restrict__ L, int m,
     for (int k = 0; k < R; ++k) o |= (uint32_t)((j >> k) & 1) << rp[k];
     roff[j] = o;
   }
+  // every position is loaded, the register bits' too: independent loads
   toff = 0;
-  uint32_t tm = ((1u << m) - 1u) & ~mask;
-  for (int i = 0; tm != 0u; ++i) {
-    toff |= (uint32_t)((tid >> i) & 1) << L[__builtin_ctz(tm)];
-    tm &= tm - 1u;
+  int i = 0;
+#pragma unroll
+  for (int q = 0; q < T_MAX + R; ++q) {
+    const uint32_t at = (uint32_t)L[q < m ? q : m - 1];
+    const bool thr = q < m && !((mask >> q) & 1u);
+    toff |= thr ? (((uint32_t)tid >> i) & 1u) << at : 0u;
+    i += thr;
   }
 }
 
 __device__ __forceinline__ uint32_t group_offset(const int* __restrict__ nlpos, int nnl, uint64_t rest) {
   uint32_t o = 0;
-  for (int i = 0; i < nnl; ++i) o |= (uint32_t)((rest >> i) & 1ull) << nlpos[i];
+  for (int i0 = 0; i0 < nnl; i0 += 8) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int i = i0 + k < nnl ? i0 + k : nnl - 1;   // past the end: the top bit once more
+      o |= (uint32_t)((rest >> i) & 1ull) << nlpos[i];
+    }
+  }
   return o;
 }
 
@@ -632,7 +684,7 @@ __global__ __launch_bounds__(512) void k_stage_fwd(float2* __restrict__ out, con
   const int* __restrict__ rpos = tpos + T;
   const int* __restrict__ nlpos = rpos + R;
   const int* __restrict__ ops = h + h[H_OFF_OPS];
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, stid = tid << (T_MAX - T);
   const int m = h[H_M];
   uint32_t toff, roff[NS], soff, sroff[NS];     // load / store layout
   layout_offsets(tpos, m, T, (h[H_FLAGS] >> FL_LOAD_SHIFT) & FL_MASK, tid, toff, roff);
@@ -655,10 +707,10 @@ __global__ __launch_bounds__(512) void k_stage_fwd(float2* __restrict__ out, con
       for (int j = 0; j < NS; ++j) a[j] = src[roff[j]];
     }
     for (int o = 0; o < n_ops; ++o) {
-      const int* __restrict__ w = ops + 8 * o;
+      const OpWords w = op_words(ops + 8 * o);
       if ((w[0] & 15) == OP_REMAP) {
         const int* rec = h + w[7];
-        remap(a, lds, rec, rec + T + R, T, tid);
+        remap(a, lds, layout_ending(rec + T + R, stid), layout_ending(rec + 2 * (T + R), stid));
         continue;
       }
       const float2* M = mats + w[1] + ((w[0] & F_BATCHED) ? (int64_t)row * w[2] : 0);
@@ -691,7 +743,7 @@ __global__ __launch_bounds__(512) void k_stage_adj(float2* __restrict__ psi, flo
   const int* __restrict__ nlpos = rpos + R;
   const int* __restrict__ ops = h + h[H_OFF_OPS];
   const int* __restrict__ gslot = h + h[H_OFF_GSLOT];
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, stid = tid << (T_MAX - T);
   const int lane = tid & 63;
   const int wwidth = blockDim.x < 64 ? (int)blockDim.x : 64;
   float* __restrict__ wacc = gacc + (tid >> 6) * n_gp;   // this wave's row
@@ -739,11 +791,12 @@ __global__ __launch_bounds__(512) void k_stage_adj(float2* __restrict__ psi, flo
       for (int j = 0; j < NS; ++j) l[j] = sl[roff[j]];
     }
     for (int o = n_ops - 1; o >= 0; --o) {
-      const int* __restrict__ w = ops + 8 * o;
+      const OpWords w = op_words(ops + 8 * o);
       if ((w[0] & 15) == OP_REMAP) {
         const int* rec = h + w[7];
-        remap(p, lds, rec + T + R, rec, T, tid);
-        remap(l, lds, rec + T + R, rec, T, tid);
+        const Layout from = layout_ending(rec + 2 * (T + R), stid), to = layout_ending(rec + T + R, stid);
+        remap(p, lds, from, to);
+        remap(l, lds, from, to);
         continue;
       }
       const float2* M = mats + w[1] + ((w[0] & F_BATCHED) ? (int64_t)row * w[2] : 0);
@@ -879,6 +932,7 @@ __device__ __forceinline__ void batch_item(float2* __restrict__ states, const Ba
   const int* __restrict__ rpos = tpos + T;
   const int* __restrict__ nlpos = rpos + R;
   const int* __restrict__ ops = h + h[H_OFF_OPS];
+  const int stid = tid << (T_MAX - T);
   const bool active = tid < (1 << T);
   uint32_t toff, roff[NS], soff, sroff[NS];   // load / store layout
   layout_offsets(tpos, h[H_M], T, (h[H_FLAGS] >> FL_LOAD_SHIFT) & FL_MASK, tid, toff, roff);
@@ -897,10 +951,10 @@ __device__ __forceinline__ void batch_item(float2* __restrict__ states, const Ba
       for (int j = 0; j < NS; ++j) a[j] = state_load<COHERENT>(src + roff[j]);
     }
     for (int o = 0; o < n_ops; ++o) {
-      const int* __restrict__ w = ops + 8 * o;
+      const OpWords w = op_words(ops + 8 * o);
       if ((w[0] & 15) == OP_REMAP) {
         const int* rec = h + w[7];
-        remap(a, lds, rec, rec + T + R, T, tid, active);
+        remap(a, lds, layout_ending(rec + T + R, stid), layout_ending(rec + 2 * (T + R), stid), active);
         continue;
       }
       fwd_op<FEAT_MAT2 | FEAT_MATK>(a, w, mats + w[1], tid);
