@@ -622,3 +622,39 @@ def test_remaps_of_every_thread_count(stage_bits):
         tq.expval_pauli_sum(q, obs, coef).sum().backward()
         grads.append(torch.cat([t.grad.reshape(-1) for t in ts]).cpu())
     assert (grads[0] - grads[1]).abs().max() < 5e-5
+
+
+@gpu
+@pytest.mark.parametrize("n,bsz", [(19, 9), (22, 2)])
+def test_grouped_values_keep_their_small_digits(n, bsz):
+    """Values near zero of large random states, where only the order and width
+    of the sums decide the error: Z strings inside a set, on the wires outside
+    it and across, with strings that flip bits.  A slot's product is rounded by
+    2^-24 of 2^-n, a few times (sums over a thread's slots and a few lanes):
+    over 2^n slots at random 2^-24 2^(-n/2) sqrt(13), times 6 for the largest
+    of the values, and 2^-24 of a value (within 6 2^(-n/2)) for the result."""
+    import torchquantum_amd as tq
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    psi = torch.randn(bsz, 1 << n, 2, device="cuda", generator=gen)
+    psi /= psi.double().square().sum((1, 2), keepdim=True).sqrt()
+    psi = torch.view_as_complex(psi.float().contiguous())
+    at = [{0: "Z"}, {1: "Z", 2: "Z"}, {n - 1: "Z"}, {0: "Z", n - 1: "Z"}, {n // 2: "Z", 3: "Z"}, {0: "X"},
+          {1: "X", 0: "Z"}, {n - 1: "X", 0: "Z", 1: "Z"}, {n // 2: "Y", n // 2 - 1: "Y"}, {0: "X", n - 2: "X", 4: "Z"}]
+    obs = ["".join(d.get(w, "I") for w in range(n)) for d in at]
+    q = tq.QuantumDevice(n_wires=n, bsz=bsz, device="cuda")
+    q.set_states(psi)
+    got = tq.expval_joint_analytical_batch(q, obs).double()
+    total = tq.expval_pauli_sum(q, obs, [1.0] * len(obs)).double()
+    wide = psi.to(torch.complex128)
+    want = []
+    for d in at:
+        x = wide.reshape([bsz] + [2] * n)
+        for w, c in d.items():
+            a, b = x.select(w + 1, 0), x.select(w + 1, 1)
+            a, b = (a, -b) if c == "Z" else (b, a) if c == "X" else (-1j * b, 1j * a)
+            x = torch.stack((a, b), w + 1)
+        want.append((wide.conj() * x.reshape(bsz, -1)).sum(1).real)
+    want = torch.stack(want, 1)
+    tol = 2.0 ** -24 * 2.0 ** (-n / 2) * (13 ** 0.5 * 6 + 6)
+    assert (got - want).abs().max() < tol
+    assert (total.reshape(-1) - want.sum(1)).abs().max() < tol * len(obs)

@@ -61,6 +61,18 @@ __device__ __forceinline__ double wave_sum_d(double v) {
   return v;
 }
 
+// The workgroup's sum in float64; red: a double of LDS per wavefront.
+__device__ __forceinline__ double block_sum_d(double v, double* red) {
+  v = wave_sum_d(v);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+  if (threadIdx.x == 0)
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += red[i];
+  return s;  // valid in thread 0
+}
+
 // Loads in flight per thread in the chunk walks below: one 16-byte load per
 // trip leaves too few bytes in flight to cover HBM latency.
 constexpr int EV_UNROLL = 4;
@@ -470,17 +482,26 @@ __device__ __forceinline__ float pg_sum16(float a, float b) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-__device__ __forceinline__ float pg_sum8(const float (&v)[8], int lane) {
+// v of the lane that DPP control C names
+template <int C>
+__device__ __forceinline__ double pg_dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), C, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), C, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+// The two steps that halve the values run in float32, the others in float64:
+// a sum over all lanes of same-signed slots (a Z string outside the lanes'
+// bits) is 64 times a lane's, and so would be the rounding of the last steps.
+__device__ __forceinline__ double pg_sum8(const float (&v)[8], int lane) {
   float w[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) w[i] = pg_sum32(v[i], v[i + 4]);
-  const float u0 = pg_sum16(w[0], w[2]), u1 = pg_sum16(w[1], w[3]);
-  const float s0 = u0 + __builtin_amdgcn_update_dpp(0.f, u0, 0x128, 0xf, 0xf, false);   // row_ror:8
-  const float s1 = u1 + __builtin_amdgcn_update_dpp(0.f, u1, 0x128, 0xf, 0xf, false);
-  float z = (lane & 8) ? s1 : s0;
-  z += __builtin_amdgcn_update_dpp(0.f, z, 0x141, 0xf, 0xf, false);   // row_half_mirror
-  z += __builtin_amdgcn_update_dpp(0.f, z, 0x4E, 0xf, 0xf, false);    // quad_perm: l ^ 2
-  z += __builtin_amdgcn_update_dpp(0.f, z, 0xB1, 0xf, 0xf, false);    // quad_perm: l ^ 1
+  const double u0 = pg_sum16(w[0], w[2]), u1 = pg_sum16(w[1], w[3]);
+  const double s0 = u0 + pg_dpp<0x128>(u0), s1 = u1 + pg_dpp<0x128>(u1);   // row_ror:8
+  double z = (lane & 8) ? s1 : s0;
+  z += pg_dpp<0x141>(z);   // row_half_mirror
+  z += pg_dpp<0x4E>(z);    // quad_perm: l ^ 2
+  z += pg_dpp<0xB1>(z);    // quad_perm: l ^ 1
   return z;
 }
 
@@ -509,8 +530,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                                                           int64_t gpw, float* __restrict__ dotpart) {
   __shared__ float2 buf[NR * NT];
   __shared__ float2 cg[PG_MAXT];        // the group's coefficients, signs of the group bits folded in
-  __shared__ float red[NT / 64];
-  float dsum = 0.f;
+  __shared__ double red[NT / 64];
+  double dsum = 0.0;
   const int tid = threadIdx.x;
   const uint32_t tsc = pg_scatter(g, (uint32_t)tid);
   uint32_t rsc[NR];
@@ -593,16 +614,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     }
     pg_store<NR, BIG>(rout, tsc, rsc, acc);
     if (dotpart) {
+      float d = 0.f;
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         const float2 v = buf[tid + r * NT];
-        dsum = fmaf(v.x, acc[r].x, fmaf(v.y, acc[r].y, dsum));
+        d = fmaf(v.x, acc[r].x, fmaf(v.y, acc[r].y, d));
       }
+      dsum += d;
     }
   }
   if (dotpart) {
-    const float t = block_sum(dsum, red);
-    if (tid == 0) dotpart[blockIdx.x] = t;
+    const double t = block_sum_d(dsum, red);
+    if (tid == 0) dotpart[blockIdx.x] = (float)t;
   }
 }
 
@@ -611,25 +634,28 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // <P> = Re(i^{nY} S), S = sum_j (-1)^{popcount(j & z)} conj(b) a, so only
 // Re S (nY even) or Im S (nY odd) is accumulated.  Per entry one sum over the
 // slots; per term the lane's sign of it, eight terms reduced over the
-// wavefront at a time into the wave's row of gacc.  Bound by the entries' LDS
+// wavefront at a time into the wave's row of gacc, in float64: a wave's sum
+// runs over many groups, and in float32 its rounding was the largest error of
+// the value (24 qubits bsz 4: 4e-6 of the values' norm, now 2e-7).  Bound by the entries' LDS
 // reads and multiply-adds: 24 qubits bsz 4 with 60 strings, 5 passes of 198 us
 // and one launch for a pass's sums (16 terms at most per set and a launch per
 // term before).
-// part[blockIdx.x * nt + t] = the partial of term t.
+// part[(blockIdx.x * nt + t) * 2] = the partial of term t, and what float32
+// leaves off it.
 template <int NT, int NR, bool BIG>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_pauli_group_expval(const float2* __restrict__ in, int n, PGroup g,
                                                            int64_t gpw, float* __restrict__ part) {
   __shared__ float2 buf[NR * NT];
-  __shared__ float gacc[NT / 64][PG_MAXT];
+  __shared__ double gacc[NT / 64][PG_MAXT];
   __shared__ uint32_t zgs[PG_MAXT];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  float* wacc = gacc[tid >> 6];
+  double* wacc = gacc[tid >> 6];
   const uint32_t tsc = pg_scatter(g, (uint32_t)tid);
   uint32_t rsc[NR];
 #pragma unroll
   for (int r = 0; r < NR; ++r) rsc[r] = pg_scatter(g, (uint32_t)r * NT);
-  for (int t = tid; t < (NT / 64) * PG_MAXT; t += NT) gacc[0][t] = 0.f;
+  for (int t = tid; t < (NT / 64) * PG_MAXT; t += NT) gacc[0][t] = 0.0;
   if (tid < g.nt) zgs[tid] = g.zg[tid];
   uint32_t lw[PG_WORDS];
   pg_lane_signs(g, (uint32_t)tid, lw);
@@ -676,23 +702,26 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         v[k] = __uint_as_float(__float_as_uint(F) ^ (w & 0x80000000u));
         w <<= 1;
       }
-      const float c = pg_sum8(v, lane);
+      const double c = pg_sum8(v, lane);
       const int t = t0 + (lane >> 3);
-      if ((lane & 7) == 0 && t < g.nt) wacc[t] += flip_sign(c, __popc(goff & zgs[t]) & 1u);
+      if ((lane & 7) == 0 && t < g.nt) wacc[t] += (__popc(goff & zgs[t]) & 1u) ? -c : c;
     }
 #pragma unroll
     for (int r = 0; r < NR; ++r) a[r] = an[r];
   }
   __syncthreads();
   for (int t = tid; t < g.nt; t += NT) {
-    float s = 0.f;
+    double s = 0.0;
     for (int w = 0; w < NT / 64; ++w) s += gacc[w][t];
-    part[(uint64_t)blockIdx.x * g.nt + t] = s;
+    float* o = part + ((uint64_t)blockIdx.x * g.nt + t) * 2;
+    const float f = (float)s;
+    o[0] = f;
+    o[1] = (float)(s - (double)f);
   }
 }
 
-// out[row * ostride + col[t]] = the sum of part[(row * nchunks + c) * nt + t]
-// over the chunks, in float64, negated where bit t of neg is set; one
+// out[row * ostride + col[t]] = the sum of the W floats at
+// part[((row * nchunks + c) * nt + t) * W] over the chunks, in float64, negated where bit t of neg is set; one
 // wavefront per (row, t).
 struct TermSums {
   int nt;
@@ -700,6 +729,7 @@ struct TermSums {
   uint32_t neg[(PG_MAXT + 31) / 32];
 };
 
+template <int W>
 __global__ __launch_bounds__(256) void k_sum_terms(const float* __restrict__ part, int nchunks, int64_t bsz,
                                                    TermSums ts, float* __restrict__ out, int64_t ostride) {
   const int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;   // wave-uniform
@@ -708,7 +738,11 @@ __global__ __launch_bounds__(256) void k_sum_terms(const float* __restrict__ par
   const int64_t row = i / ts.nt;
   const int t = (int)(i - row * ts.nt);
   double s = 0.0;
-  for (int c = lane; c < nchunks; c += 64) s += part[(row * nchunks + c) * ts.nt + t];
+  for (int c = lane; c < nchunks; c += 64) {
+    const float* p = part + ((row * nchunks + c) * ts.nt + t) * W;
+#pragma unroll
+    for (int k = 0; k < W; ++k) s += p[k];
+  }
   s = wave_sum_d(s);
   if (lane == 0) out[row * ostride + ts.col[t]] = (float)((ts.neg[t >> 5] >> (t & 31)) & 1u ? -s : s);
 }
@@ -769,7 +803,7 @@ static int pg_expval_launch(hipStream_t s, const float2* in, int n, const PGroup
   wpr = pg_wg_per_row(bsz, g.nnl, g.m);
   const int64_t gpw = per_row / wpr;
   const int64_t grid = bsz * wpr;
-  if (grid > 0x7fffffffll || ws_bytes < grid * g.nt * (int64_t)sizeof(float)) return 1;   // caller falls back
+  if (grid > 0x7fffffffll || ws_bytes < grid * 2 * g.nt * (int64_t)sizeof(float)) return 1;   // caller falls back
   return pg_dispatch(g, [&](auto nt, auto nr, auto big) {
     k_pauli_group_expval<nt(), nr(), big()><<<(unsigned)grid, nt(), 0, s>>>(in, n, g, gpw, (float*)ws);
     return check_launch("tqsv_expval_pauli/group");
@@ -1036,7 +1070,7 @@ TQSV_API int tqsv_expval_pauli(hipStream_t s, const void* state, int64_t bsz, in
         if ((ny & 3) == 1 || (ny & 3) == 2) ts.neg[q >> 5] |= 1u << (q & 31);
         done[t] = 1;
       }
-      k_sum_terms<<<sum_grid(bsz * g.nt), 256, 0, s>>>((const float*)workspace, (int)wpr, bsz, ts, out, out_stride);
+      k_sum_terms<2><<<sum_grid(bsz * g.nt), 256, 0, s>>>((const float*)workspace, (int)wpr, bsz, ts, out, out_stride);
       if ((rc = check_launch("tqsv_expval_pauli/groupsum"))) return rc;
     }
   }
@@ -1055,7 +1089,7 @@ TQSV_API int tqsv_expval_pauli(hipStream_t s, const void* state, int64_t bsz, in
     int rc = check_launch("tqsv_expval_pauli/diag");
     if (rc) return rc;
     ts.nt = zm.nt;
-    k_sum_terms<<<sum_grid(bsz * ts.nt), 256, 0, s>>>((const float*)workspace, (int)nchunks, bsz, ts, out, out_stride);
+    k_sum_terms<1><<<sum_grid(bsz * ts.nt), 256, 0, s>>>((const float*)workspace, (int)nchunks, bsz, ts, out, out_stride);
     if ((rc = check_launch("tqsv_expval_pauli/sum"))) return rc;
   }
   for (int t = 0; t < nterms; ++t) {
