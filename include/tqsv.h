@@ -112,6 +112,8 @@ int tqsv_jit_compile(const char* src, const char* opts, void* code, int64_t cap,
 /* load a code object on the current device; funcs[i] = kernel names[i]. */
 int tqsv_jit_load(const void* code, int64_t size, int n, const char* const* names, void** module, void** funcs);
 int tqsv_jit_unload(void* module);
+/* *bytes = scratch memory per thread of a loaded kernel (what it spills). */
+int tqsv_jit_scratch_bytes(const void* func, int* bytes);
 /* func: kernel compiled from prog_host's program (parameters: out, in, mats,
  * init_zero, n_groups, groups_per_wg). */
 int tqsv_jit_stage_forward(tqsv_stream_t s, const void* func, void* state_out, const void* state_in, int64_t bsz,

@@ -206,3 +206,25 @@ def test_jit_auto_compiles_in_background():
     assert any(c._jit.get("f") for c in plans) and any(c._jit.get("a") for c in plans)
     assert np.abs(outs[0][0] - outs[1][0]).max() < 1e-6
     assert np.abs(outs[0][1] - outs[1][1]).max() < 1e-5
+
+
+@gpu
+@pytest.mark.parametrize("limit", [-1, 1 << 20])
+def test_jit_forward_kernels_held_and_not_held(limit, monkeypatch):
+    """13-bit stages whose kernels are all compiled again without the register
+    limit (limit -1) or all keep it, whatever they spill: the same arithmetic,
+    so the bars of the other cases."""
+    from torchquantum_amd import engine as E, stagejit as J
+    monkeypatch.setattr(J, "FWD_SCRATCH", limit)
+    E._plan_cache.clear()
+    rng = np.random.default_rng(5)
+    n, bsz = 15, 2
+    ops = random_ops(n, 120, bsz, rng, names=["rx", "ry", "rz", "u3", "cnot"])
+    got = _run(n, bsz, ops, jit="on", stage_bits=13)
+    plans = _plans_with_jit("f")
+    assert plans, "compiled stage kernels did not run"
+    if limit < 0:
+        assert all(J._scratch_bytes(f) == 0 for c in plans for f in c._jit["f"].values())
+    interp = _run(n, bsz, ops, jit="off", stage_bits=13)
+    assert np.abs(got - O.run_ops(oracle_ops(ops, bsz), n, bsz)).max() < 1e-5
+    assert np.abs(got - interp).max() < 1e-6

@@ -72,6 +72,7 @@ SIGNATURES = {
     "tqsv_jit_load": (c_int, [c_void_p, c_int64, c_int, POINTER(ctypes.c_char_p), POINTER(c_void_p),
                               POINTER(c_void_p)]),
     "tqsv_jit_unload": (c_int, [c_void_p]),
+    "tqsv_jit_scratch_bytes": (c_int, [c_void_p, c_int_p]),
     "tqsv_jit_stage_forward": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int_p, c_void_p,
                                        c_int, c_int]),
     "tqsv_jit_stage_adjoint": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int,

@@ -130,6 +130,13 @@ TQSV_API int tqsv_jit_unload(void* module) {
   return OK;
 }
 
+TQSV_API int tqsv_jit_scratch_bytes(const void* func, int* bytes) {
+  if (!func || !bytes) { set_error("tqsv_jit_scratch_bytes: null argument"); return E_ARG; }
+  hipError_t e = hipFuncGetAttribute(bytes, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, (hipFunction_t)const_cast<void*>(func));
+  if (e != hipSuccess) { set_error("tqsv_jit_scratch_bytes: %s", hipGetErrorString(e)); return E_LAUNCH; }
+  return OK;
+}
+
 // One stage of a forward pass with a compiled stage kernel.  Arguments as
 // tqsv_stage_forward; func: the kernel compiled from the same program
 // (kernel parameters: out, in, mats, init_zero, n_groups, groups_per_wg).

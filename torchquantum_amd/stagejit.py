@@ -51,9 +51,14 @@ COMPILE_OPTS = {"f": "", "a": "-mllvm -amdgpu-sched-strategy=iterative-maxocc"}
 # local bits, four 256-thread ones with 12), but LLVM takes 130-140 VGPRs for
 # some 13-bit stages, which leaves one workgroup per CU and nothing to run
 # while it waits at a remap barrier.  Measured over the 30-qubit bsz-4 layer
-# circuit (35 stages): 632.7 -> 583.3 ms.  12-bit stages stay below 128 by themselves
-# (20 qubits bsz 16: unchanged).
+# circuit (35 stages): 632.7 -> 583.3 ms.  12-bit stages stay below 128 by
+# themselves (20 qubits bsz 16: unchanged).  A stage that takes 156 and more
+# spills when held: one with 44 bytes a thread ran in 4.4 instead of 3.9 ms,
+# with 92 bytes in 6.2 instead of 4.4 (24 qubits bsz 64), while up to 20 bytes
+# cost less than the second workgroup gains.  So a kernel that spills more than
+# FWD_SCRATCH bytes is compiled again without the limit.
 FWD_WAVES_PER_EU = 4
+FWD_SCRATCH = 32
 COMPILE_OPTS["p"] = COMPILE_OPTS["a"]     # pruned adjoint stages (gen_adjoint with skip / no_store)
 # Code-generation defaults (gen_forward / gen_adjoint arguments of the same
 # names), chosen by timing the stages of the 24-qubit bsz-64 gradient on
@@ -987,14 +992,15 @@ def _codegen(buf: Optional[bool], prefetch: Optional[bool], kind: str, lds: Opti
 
 def gen_forward(words: np.ndarray, name: str, nontemporal: bool = False, buf: Optional[bool] = None,
                 prefetch: Optional[bool] = None, lds: Optional[str] = None, mfma: Optional[bool] = None,
-                lane_remap: Optional[bool] = None) -> str:
+                lane_remap: Optional[bool] = None, waves: int = FWD_WAVES_PER_EU) -> str:
     """HIP source of one forward stage kernel (k_stage_fwd semantics).
     nontemporal: the state is read and written with non-temporal hints;
     buf: buffer instructions for the state where the offsets allow;
     prefetch: each group's loads are issued one group ahead (software
     pipelining), so that they are in flight while the previous group
     computes; lds: the remap buffer's index map, "xor" (swizzled) or "pad4" /
-    "pad5" (padded, additive).  None takes the module default (CODEGEN)."""
+    "pad5" (padded, additive).  None takes the module default (CODEGEN).
+    waves: wavefronts per SIMD that the registers must allow (0: no limit)."""
     sp = StageProgram(words)
     if sp.T < MIN_T:
         raise ValueError("compiled stages need T >= 6")
@@ -1011,8 +1017,8 @@ def gen_forward(words: np.ndarray, name: str, nontemporal: bool = False, buf: Op
     body = ["  " + s for s in g.lines]
     stores = [f"      {_store(sp, 'out', j, a[j], mode, lay='st')}" for j in range(NS)]
     nt = 1 << sp.T
-    src = [f'extern "C" __global__ void __launch_bounds__({nt}) '
-           f'__attribute__((amdgpu_waves_per_eu({FWD_WAVES_PER_EU}))) {name}(float2* __restrict__ out, '
+    held = f"__attribute__((amdgpu_waves_per_eu({waves}))) " if waves else ""
+    src = [f'extern "C" __global__ void __launch_bounds__({nt}) {held}{name}(float2* __restrict__ out, '
            "const float2* __restrict__ in, const float2* __restrict__ mats, int init_zero, long long n_groups, "
            "long long gpw) {"]
     if g.used_lds:
@@ -1219,7 +1225,7 @@ def kernel_name(kind: str, prog, nt: bool = False) -> str:
         hs.update(repr(sorted(extra.items())).encode())
     hs.update(COMPILE_OPTS[kind].encode())
     if kind == "f":
-        hs.update(f"w{FWD_WAVES_PER_EU}".encode())
+        hs.update(f"w{FWD_WAVES_PER_EU},{FWD_SCRATCH}".encode())
     hs.update(repr((_codegen(None, None, kind), _mfma(kind), _lane(kind))).encode())
     if nt:
         hs.update(b"nt")
@@ -1317,36 +1323,60 @@ def get_kernels(programs: Sequence[np.ndarray], kind: str, device_index: int, nt
             if (device_index, nm) not in _funcs and nm not in missing:
                 missing[nm] = w
     if missing:
-        items = list(missing.items())
-        chunks = [items[i:i + KERNELS_PER_SOURCE] for i in range(0, len(items), KERNELS_PER_SOURCE)]
-        codes = []
-        verbose = os.environ.get("TQSV_JIT_LOG") == "1"
-        for ci, ch in enumerate(chunks):
-            if _shutdown.is_set():
-                raise RuntimeError("stage kernel compile cancelled at interpreter exit")
-            codes.append(compile_source(PRELUDE + (NT_HELPERS if nt else "") + "\n".join(gen(w, nm, nt) for nm, w in ch),
-                                        COMPILE_OPTS[kind]))
-            if verbose:
-                import sys
-                print(f"[stagejit] {kind}: {min((ci + 1) * KERNELS_PER_SOURCE, len(items))}/{len(items)} stage "
-                      "kernels compiled", file=sys.stderr, flush=True)
-        lib = N.lib()
+        built = _build(missing, gen, kind, nt)
+        if kind == "f":
+            spilled = {nm: missing[nm] for nm, f in built.items() if _scratch_bytes(f) > FWD_SCRATCH}
+            if spilled:
+                built.update(_build(spilled, lambda w, nm, nt: gen_forward(w, nm, nt, waves=0), kind, nt))
         with _lock:
-            for ch, code in zip(chunks, codes):
-                if all((device_index, nm) in _funcs for nm, _ in ch):
-                    continue
-                cnames = (ctypes.c_char_p * len(ch))(*[nm.encode() for nm, _ in ch])
-                fptrs = (ctypes.c_void_p * len(ch))()
-                mod = ctypes.c_void_p()
-                buf = ctypes.create_string_buffer(code, len(code))
-                rc = lib.tqsv_jit_load(buf, len(code), len(ch), cnames, ctypes.byref(mod), fptrs)
-                if rc != 0:
-                    raise RuntimeError(f"stage kernel load failed: {lib.tqsv_last_error().decode(errors='replace')}")
-                _modules.append(mod.value)
-                for (nm, _), f in zip(ch, fptrs):
-                    _funcs[(device_index, nm)] = f
+            for nm, f in built.items():
+                _funcs.setdefault((device_index, nm), f)
     with _lock:
         return [_funcs[(device_index, nm)] for nm in names]
+
+
+def _build(programs: Dict[str, np.ndarray], gen, kind: str, nt: bool) -> Dict[str, int]:
+    """Compiles and loads (on the current device) the kernels gen(program,
+    name, nt); name -> hipFunction_t."""
+    from . import _native as N
+    items = list(programs.items())
+    chunks = [items[i:i + KERNELS_PER_SOURCE] for i in range(0, len(items), KERNELS_PER_SOURCE)]
+    codes = []
+    verbose = os.environ.get("TQSV_JIT_LOG") == "1"
+    for ci, ch in enumerate(chunks):
+        if _shutdown.is_set():
+            raise RuntimeError("stage kernel compile cancelled at interpreter exit")
+        codes.append(compile_source(PRELUDE + (NT_HELPERS if nt else "") + "\n".join(gen(w, nm, nt) for nm, w in ch),
+                                    COMPILE_OPTS[kind]))
+        if verbose:
+            import sys
+            print(f"[stagejit] {kind}: {min((ci + 1) * KERNELS_PER_SOURCE, len(items))}/{len(items)} stage "
+                  "kernels compiled", file=sys.stderr, flush=True)
+    lib = N.lib()
+    out: Dict[str, int] = {}
+    with _lock:
+        for ch, code in zip(chunks, codes):
+            cnames = (ctypes.c_char_p * len(ch))(*[nm.encode() for nm, _ in ch])
+            fptrs = (ctypes.c_void_p * len(ch))()
+            mod = ctypes.c_void_p()
+            buf = ctypes.create_string_buffer(code, len(code))
+            rc = lib.tqsv_jit_load(buf, len(code), len(ch), cnames, ctypes.byref(mod), fptrs)
+            if rc != 0:
+                raise RuntimeError(f"stage kernel load failed: {lib.tqsv_last_error().decode(errors='replace')}")
+            _modules.append(mod.value)
+            for (nm, _), f in zip(ch, fptrs):
+                out[nm] = f
+    return out
+
+
+def _scratch_bytes(func: int) -> int:
+    """Bytes a thread of a loaded kernel spills to memory."""
+    from . import _native as N
+    size = ctypes.c_int(0)
+    lib = N.lib()
+    if lib.tqsv_jit_scratch_bytes(func, ctypes.byref(size)) != 0:
+        raise RuntimeError(f"stage kernel query failed: {lib.tqsv_last_error().decode(errors='replace')}")
+    return size.value
 
 
 # ----------------------------------------------------------------------------
