@@ -771,3 +771,27 @@ def test_swaps_move_no_data_inside_a_stage(n, stage_bits, io):
                                E.Compiled(tape, n, bsz, E.EngineOptions(mode="pergate", adjoint_mg=False), "cpu")
                                .pool_host(tape, True, True).astype(np.complex128), psi.copy(), cvec.copy())
     assert np.abs(full[:, :c.n_slots] - want[:, :c.n_slots]).max() < 1e-5 * (1 + np.abs(want).max())
+
+
+def test_learned_planner_keeps_the_default_beyond_what_it_saw():
+    """Plans that fill the chip, when no timed plan did, take the first candidate; all others the smallest
+    prediction.  (A stub in place of the network: the rule alone.)"""
+    from torchquantum_amd.autotune import LearnedPlanner
+    from torchquantum_amd.costmodel import FEATURES, MLPCostModel
+
+    class Stub(MLPCostModel):
+        def __init__(self, max_groups):
+            self.max_groups = max_groups
+
+        def predict_ms(self, X):
+            return -np.arange(len(X), dtype=np.float64)     # the last candidate is best
+
+    def records(n, m):
+        f = [0.0] * len(FEATURES)
+        f[0], f[14] = float(n), float(m)
+        return [{"features": f, "opts": {"fusion_width": k}} for k in (1, 2, 3)]
+
+    for max_groups, n, m, width in ((256.0, 20, 12, 3), (256.0, 21, 12, 1), (1.0, 12, 12, 3), (1.0, 16, 12, 1),
+                                    (1024.0, 30, 12, 3), (None, 30, 12, 3), (256.0, 25, 0, 3)):
+        pick = LearnedPlanner(Stub(max_groups)).choose_from_records(records(n, m))
+        assert pick.fusion_width == width, (max_groups, n, m)

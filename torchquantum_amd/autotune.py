@@ -108,13 +108,15 @@ class Autotuner:
 
 
 class LearnedPlanner:
-    """Pick the candidate with the smallest predicted time (no launches)."""
+    """Pick the candidate with the smallest predicted time (no launches).
+    For a circuit whose stages fill the chip, when no timed one's did, the
+    first candidate is taken (MLPCostModel.covers)."""
 
     def __init__(self, model: MLPCostModel, candidates: Sequence[E.EngineOptions] = DEFAULT_CANDIDATES):
         self.model = model
         self.candidates = list(candidates)
 
-    def score(self, tape, n, bsz):
+    def _score(self, tape, n, bsz):
         opts, feats = [], []
         for o in self.candidates:
             o = E.EngineOptions(**{**o.__dict__, "stage_bits": min(o.stage_bits or 12, n)})
@@ -124,17 +126,21 @@ class LearnedPlanner:
             opts.append(o)
             feats.append(plan_features(c))
         pred = self.model.predict_ms(np.array(feats))
-        return opts, pred
+        return opts, pred, self.model.covers(np.array(feats))
+
+    def score(self, tape, n, bsz):
+        return self._score(tape, n, bsz)[:2]
 
     def choose(self, tape, n, bsz) -> E.EngineOptions:
-        opts, pred = self.score(tape, n, bsz)
-        return opts[int(np.argmin(pred))]
+        opts, pred, known = self._score(tape, n, bsz)
+        return opts[int(np.argmin(pred)) if known else 0]
 
     def choose_from_records(self, records: Sequence[dict]) -> E.EngineOptions:
         """The candidate with the smallest predicted time among an autotuner
         entry's records, from their stored plan features (no plan rebuilt)."""
-        pred = self.model.predict_ms(np.array([r["features"] for r in records]))
-        return E.EngineOptions(**records[int(np.argmin(pred))]["opts"])
+        feats = np.array([r["features"] for r in records])
+        best = int(np.argmin(self.model.predict_ms(feats))) if self.model.covers(feats) else 0
+        return E.EngineOptions(**records[best]["opts"])
 
 
 def tune_circuits(tuner: "Autotuner", tapes: Sequence[tuple], candidates: Sequence[E.EngineOptions],

@@ -26,6 +26,9 @@ FEATURES = ["log2_amps", "n_qubits", "log2_bsz", "stages", "solos", "ops", "mat1
 _OP_FLOPS = {"mat1": 16.0, "mat2": 32.0, "matk": 128.0, "diag": 8.0, "swap": 2.0}
 
 
+CUS = 256     # compute units of an MI355X
+
+
 def plan_features(c: E.Compiled) -> np.ndarray:
     n, bsz = c.n, c.bsz
     amps = float(bsz) * (1 << n)
@@ -73,6 +76,7 @@ class MLPCostModel:
         self.t = 0
         self.mu = None
         self.sd = None
+        self.max_groups: Optional[float] = None
         self.x_min = None
         self.x_max = None
         self.y_mu = 0.0
@@ -149,6 +153,20 @@ class MLPCostModel:
         return torch.tensor(Z, dtype=torch.float32, device=self.device)
 
     @staticmethod
+    def groups(X: np.ndarray) -> np.ndarray:
+        """Workgroup-sized pieces a stage of each plan has to work on."""
+        X = np.atleast_2d(np.asarray(X, dtype=np.float64))
+        return np.where(X[:, 14] > 0, np.exp2(X[:, 0] - X[:, 14]), 1.0)
+
+    def covers(self, X: np.ndarray) -> bool:
+        """Whether the timings the model learned from say something about
+        plans of this size.  Up to one group per CU an operation costs its
+        latency, beyond that its arithmetic, and plans rank differently:
+        with circuits of at most 20 qubits timed (256 groups, fusion width 2
+        ahead by 3-13%), width 2 was 8-10% slower than width 1 at 21 and 22."""
+        return self.max_groups is None or self.max_groups > CUS or float(self.groups(X).max()) <= self.max_groups
+
+    @staticmethod
     def _log_amps(X: np.ndarray) -> np.ndarray:
         """ln(amplitudes) of each plan (feature 0 is log2 of the state size)."""
         return np.asarray(X, dtype=np.float64)[:, 0] * math.log(2.0)
@@ -163,6 +181,7 @@ class MLPCostModel:
         self.mu = X.mean(0)
         self.sd = X.std(0) + 1e-6
         self.x_min, self.x_max = X.min(0), X.max(0)
+        self.max_groups = float(self.groups(X).max()) if X.shape[1] == len(FEATURES) else None
         self.y_mu, self.y_sd = float(y.mean()), float(y.std() + 1e-6)
         Xt = self._std(X)
         yt = torch.tensor((y - self.y_mu) / self.y_sd, dtype=torch.float32, device=self.device)
