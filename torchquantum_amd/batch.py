@@ -172,10 +172,11 @@ class CircuitBatch:
         idle, and the deepest circuit's stages, each waiting for the one
         before, one after another on few of them.  So: as many groups as give
         a mean level about 1536 items, at most 6 (a claim of an item costs
-        about 50 ns on one counter), and at least 4 items per stage.  Measured, 1 / 2 / 4 / 8 groups for all: 64 circuits of
-        up to 22 qubits 11.5 / 6.8 / 6.0 / 7.1 ms, 256 of them 34.9 / 20.1 /
-        17.0 / 17.1 ms, 20 of up to 20 qubits 1.17 / 1.10 / 1.64 / 3.0 ms, 30
-        of up to 14 qubits 0.31 / 0.53 / 0.98 / 0.97 ms."""
+        about 50 ns on one counter), and at least 4 items per stage.  Measured,
+        1 / 2 / 4 / 6 groups for all: 64 circuits of up to 22 qubits 12.0 / 6.8
+        / 5.5 / 5.7 ms, 256 of them 36.5 / 19.4 / 15.0 / 14.7 ms, 20 of up to
+        20 qubits 1.16 / 1.00 / 1.38 / 1.93 ms, 30 of up to 14 qubits 0.28 /
+        0.47 / 0.83 / 0.84 ms."""
         groups = [[1 << (n - m) for m in ms] for n, ms in zip(self.ns, self.stage_m)]
         mean = sum(map(sum, groups)) / max(map(len, groups))
         most = max(1, min(6, round(mean / 1536)))
