@@ -149,6 +149,11 @@ int tqsv_adjoint_diag(tqsv_stream_t s, void* psi, void* lam, int64_t bsz, int n,
 int64_t tqsv_adjoint_work_floats(int64_t bsz, int n);
 
 /* ---- gate matrices from device parameters ------------------------------- */
+/* A host array (a multiple of 4 bytes) to device memory through kernel
+ * arguments, which a captured graph keeps: a replay writes what was passed at
+ * capture.  For streams under capture (a copy from a reused staging buffer
+ * would be made again at every replay); a launch per 3840 bytes. */
+int tqsv_put(tqsv_stream_t s, void* dst, const void* src_host, int64_t bytes);
 /* sizeof(DevOp) | sizeof(DevMember) << 16 (layouts checked by the host). */
 int tqsv_dev_gate_bytes(void);
 /* Write the matrix-pool blocks (U, dU/dtheta_p, U^dagger) of single-wire ops

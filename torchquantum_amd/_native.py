@@ -63,6 +63,7 @@ SIGNATURES = {
     "tqsv_batch_zcirc_bytes": (c_int, []),
     "tqsv_batch_zexpval": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_float_p, c_float_p]),
     "tqsv_mg_item_bytes": (c_int, []),
+    "tqsv_put": (c_int, [c_void_p, c_void_p, c_void_p, c_int64]),
     "tqsv_dev_gate_bytes": (c_int, []),
     "tqsv_build_dev_gates": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64]),
     "tqsv_mg_to_grad": (c_int, [c_void_p, c_float_p, c_int64, c_int64, c_void_p, c_int, c_void_p]),

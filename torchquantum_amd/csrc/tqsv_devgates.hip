@@ -16,6 +16,8 @@
 //   dense 2x2 ops:  [U (4), D_0 (4), ..., D_{P-1} (4)] complex per row;
 //   diagonal ops:   [U[a][a], U[b][b], D_0[a][a], D_0[b][b], ...] per row;
 //   and U^dagger (or the conjugated diagonal) at the op's adjoint block.
+#include <cstring>
+
 #include "tqsv_common.h"
 
 namespace tqsv {
@@ -247,9 +249,39 @@ __global__ void k_build_dev_gates(float2* __restrict__ pool, const DevOp* __rest
   }
 }
 
+// Host words as a kernel argument: a launch that a HIP graph records keeps its
+// arguments, so a replay writes what was passed then, whatever has become of
+// the host memory.  Below the 4096 bytes that a launch's arguments may take.
+constexpr int PUT_WORDS = 960;
+struct PutWords {
+  uint32_t w[PUT_WORDS];
+};
+
+__global__ __launch_bounds__(64) void k_put(uint32_t* __restrict__ dst, PutWords p, int n) {
+  for (int i = threadIdx.x; i < n; i += 64) dst[i] = p.w[i];
+}
+
 }  // namespace tqsv
 
 using namespace tqsv;
+
+// A host array to device memory through launch arguments (see PUT_WORDS): for
+// streams under capture, where a copy from host memory would be made again at
+// every replay.  A launch per 3840 bytes.
+TQSV_API int tqsv_put(hipStream_t s, void* dst, const void* src_host, int64_t bytes) {
+  if (!dst || !src_host || bytes < 0 || (bytes & 3)) { set_error("tqsv_put: bad arguments"); return E_ARG; }
+  for (int64_t done = 0; done < bytes;) {
+    PutWords p;
+    const int64_t left = bytes - done;
+    const int n = (int)(left < (int64_t)sizeof(p) ? left : (int64_t)sizeof(p)) / 4;
+    std::memcpy(p.w, (const char*)src_host + done, (size_t)n * 4);
+    k_put<<<1, 64, 0, s>>>((uint32_t*)((char*)dst + done), p, n);
+    const int rc = check_launch("tqsv_put");
+    if (rc) return rc;
+    done += (int64_t)n * 4;
+  }
+  return OK;
+}
 
 TQSV_API int tqsv_dev_gate_bytes(void) { return (int)sizeof(DevOp) | ((int)sizeof(DevMember) << 16); }
 

@@ -739,6 +739,25 @@ def upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
     return ring.upload(host, device)
 
 
+def _capturing(device: torch.device) -> bool:
+    """Whether the device's current stream is recording a graph."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
+def put(host: np.ndarray, device: torch.device) -> torch.Tensor:
+    """Copy of a complex64 array on the device for a stream under capture: the
+    values travel as kernel arguments, which belong to the graph.  A copy from
+    the ring would be made again at every replay, from a buffer that later
+    uploads have refilled."""
+    host = np.ascontiguousarray(host, dtype=np.complex64)
+    out = torch.empty(host.shape, dtype=torch.complex64, device=device)
+    N.call("tqsv_put", N.stream_of(out), out.data_ptr(), host.ctypes.data, host.nbytes)
+    return out
+
+
 def _host_params(tape: Sequence[TapeOp], skip: frozenset = frozenset()) -> List[Optional[np.ndarray]]:
     """Parameter values of every tape op as numpy (float64 or complex128),
     except the ops in ``skip`` (their matrices are built on the GPU).  GPU
@@ -1653,7 +1672,8 @@ class Compiled:
         host = self.pool_host(tape, with_grad, with_adj)
         if torch.device(self.device).type != "cuda":
             return torch.from_numpy(host).to(self.device)
-        pool = upload(host, torch.device(self.device))
+        device = torch.device(self.device)
+        pool = (put if _capturing(device) else upload)(host, device)
         if len(self.dev_ops):
             _check_dev_layout()
             base = pool.data_ptr() + 8 * self.pool_len
