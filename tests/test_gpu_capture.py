@@ -70,3 +70,29 @@ def test_captured_circuit(mode, n, rows):
         got = out.clone()
         assert torch.equal(got, run()), k
         assert np.isfinite(got.cpu().numpy()).all()
+
+
+@gpu
+def test_pauli_sums_of_a_given_state_are_refused():
+    """Coefficients and index tables come from host memory: their copies are refused while a graph is recorded, as
+    torch refuses a copy from pageable memory, and work after the recording as before."""
+    n = 9
+    strings, coef = ["XZ" + "I" * (n - 2), "I" * (n - 1) + "Z"], [0.5, -1.5]
+    q = tq.QuantumDevice(n_wires=n, bsz=2, device=DEV)
+    d = tq.NoiseDevice(n_wires=4, bsz=2, device=DEV)
+    for w in range(n):
+        tqf.ry(q, w, params=torch.tensor([[0.3 + w]], device=DEV))
+        if w < 4:
+            tqf.ry(d, w, params=torch.tensor([[0.3 + w]], device=DEV))
+    st = q.get_states_1d().detach()
+    calls = [lambda: tq.expval_pauli_sum(q, strings, coef),
+             lambda: tq.expval_joint_analytical(d, "XZIY"),
+             lambda: torch.autograd.grad(tq.autograd.expval_pauli_strings(st.requires_grad_(), n, strings).sum(), st)[0]]
+    want = [f().clone() for f in calls]
+    for f in calls:
+        with pytest.raises(RuntimeError, match="captured"):
+            with torch.cuda.graph(torch.cuda.CUDAGraph()):
+                f()
+    for _ in range(10):              # every buffer of the ring is still in use
+        for f, w in zip(calls, want):
+            assert torch.equal(f(), w)

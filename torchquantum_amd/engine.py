@@ -725,26 +725,30 @@ def _check_dev_layout():
         _DEV_LAYOUT_OK = True
 
 
-def upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
-    """Copy of a complex64, float32 or int64 array on the device, enqueued on
-    the current stream without waiting for the work already there (a copy
-    from pageable memory, as ``torch.tensor(..., device=)`` makes, waits)."""
-    if device.type != "cuda" or host.size == 0:
-        return torch.from_numpy(host).to(device)
-    if device.index is None:
-        device = torch.device("cuda", torch.cuda.current_device())
-    ring = _RINGS.get(device)
-    if ring is None:
-        ring = _RINGS.setdefault(device, _PinnedRing())
-    return ring.upload(host, device)
-
-
 def _capturing(device: torch.device) -> bool:
     """Whether the device's current stream is recording a graph."""
     if device.index is None or device.index == torch.cuda.current_device():
         return torch.cuda.is_current_stream_capturing()
     with torch.cuda.device(device):
         return torch.cuda.is_current_stream_capturing()
+
+
+def upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
+    """Copy of a complex64, float32 or int64 array on the device, enqueued on
+    the current stream without waiting for the work already there (a copy
+    from pageable memory, as ``torch.tensor(..., device=)`` makes, waits).
+    Refused on a stream under capture, as torch refuses the pageable copy: a
+    replay would copy whatever later uploads have put into the buffer."""
+    if device.type != "cuda" or host.size == 0:
+        return torch.from_numpy(host).to(device)
+    if _capturing(device):
+        raise RuntimeError("a copy from a shared host buffer cannot be captured into a graph")
+    if device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    ring = _RINGS.get(device)
+    if ring is None:
+        ring = _RINGS.setdefault(device, _PinnedRing())
+    return ring.upload(host, device)
 
 
 def put(host: np.ndarray, device: torch.device) -> torch.Tensor:
