@@ -867,18 +867,19 @@ __global__ __launch_bounds__(256) void k_stagepart_reduce(const float* __restric
                                                           float* __restrict__ grad, int64_t gstride) {
   const int n_gp = prog[H_NGP], nnl = prog[H_NNL];
   const int* __restrict__ gslot = prog + prog[H_OFF_GSLOT];
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;   // wave-uniform
   const int lane = threadIdx.x & 63;
-  if (i >= bsz * n_gp) return;
-  const int64_t row = i / n_gp;
-  const int t = (int)(i - row * n_gp);
-  const int64_t w0 = (row << nnl) / gpw;
-  int64_t w1 = (((row + 1) << nnl) - 1) / gpw;
-  if (w1 > grid - 1) w1 = grid - 1;
-  float s = 0.f;
-  for (int64_t w = w0 + lane; w <= w1; w += 64) s += part[(w * rpw + row - ((w * gpw) >> nnl)) * n_gp + t];
-  s = wave_sum(s);
-  if (lane == 0) grad[row * gstride + gslot[t]] += s;
+  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < bsz * n_gp; i += waves) {   // wave-uniform
+    const int64_t row = i / n_gp;
+    const int t = (int)(i - row * n_gp);
+    const int64_t w0 = (row << nnl) / gpw;
+    int64_t w1 = (((row + 1) << nnl) - 1) / gpw;
+    if (w1 > grid - 1) w1 = grid - 1;
+    float s = 0.f;
+    for (int64_t w = w0 + lane; w <= w1; w += 64) s += part[(w * rpw + row - ((w * gpw) >> nnl)) * n_gp + t];
+    s = wave_sum(s);
+    if (lane == 0) grad[row * gstride + gslot[t]] += s;
+  }
 }
 
 // ------------------------------------------------------------------ batch
@@ -1232,8 +1233,9 @@ int stage_adjoint_reduce(hipStream_t s, const int* prog_host, const int* prog_de
                          int grid, const float* work, float* grad, int64_t grad_stride) {
   const int ngp = prog_host[H_NGP];
   if (ngp == 0) return OK;
-  const int64_t waves = bsz * ngp;
-  k_stagepart_reduce<<<(unsigned)((waves + 3) / 4), 256, 0, s>>>(
+  int64_t blocks = (bsz * ngp + 3) / 4;
+  if (blocks > (1ll << 20)) blocks = 1ll << 20;   // a launch takes 2^32 threads at most; the kernel strides
+  k_stagepart_reduce<<<(unsigned)blocks, 256, 0, s>>>(
       work, prog_dev, bsz, gpw, grid, stage_rows_per_wg(prog_host, gpw), grad, grad_stride);
   return OK;
 }
