@@ -42,3 +42,40 @@ def test_gradients_of_many_rows():
     want = grads(psi[some].contiguous(), lam[some].contiguous(), mode="pergate")
     assert (got[some] - want).abs().max() < 5e-5
     assert bool((got != 0).any(1).all())            # no row left out
+
+
+@gpu
+def test_pauli_values_of_many_rows():
+    """90 strings of 8 wires in one pass and 2^26 / 90 rows and one: values and gradients of rows in every part of
+    the batch against the oracle.  Unit states, sums over 256 amplitudes: 1e-5 as in the parity tests."""
+    import torchquantum_amd as tq
+    from oracle import statevector as O
+    n, rows = 8, (1 << 26) // 90 + 1
+    rng = np.random.default_rng(6)
+    strings = sorted({"".join(rng.choice(list("IXYZ"), n)) for _ in range(120)})[:90]
+    st = _unit_rows(rows, n, 3).requires_grad_()
+    some = [0, 1, rows // 2, rows - 2, rows - 1]
+    v = st[some].detach().cpu().numpy().astype(np.complex128)
+    want = np.stack([O.expval_pauli(v, s) for s in strings], axis=1)
+    got = tq.autograd.expval_pauli_strings(st, n, strings)
+    assert np.abs(got[some].detach().cpu().numpy() - want).max() < 1e-5
+    total = tq.autograd.expval_pauli_sum_state(st, n, strings, [1.0 / 90] * 90)
+    assert np.abs(total[some].detach().cpu().numpy() - want.mean(1)).max() < 1e-5
+    (g,) = torch.autograd.grad(total.sum(), st)
+    # <P> is quadratic: Re <psi | gradient> = 2 <P>
+    dot = (st.detach().conj() * g).sum(1).real / 2
+    assert (dot - total.detach()).abs().max() < 1e-5
+
+
+@gpu
+def test_z_values_of_many_rows():
+    """<Z> of every wire for 2^24 rows and one of 4 wires, against |psi|^2 in float64."""
+    import torchquantum_amd as tq
+    n, rows = 4, (1 << 24) + 1
+    st = _unit_rows(rows, n, 4)
+    got = tq.autograd.ExpvalZAll.apply(st, n)
+    sign = torch.tensor([[1.0 - 2.0 * (j >> (n - 1 - w) & 1) for w in range(n)] for j in range(1 << n)],
+                        dtype=torch.float64, device=DEV)
+    for r0 in range(0, rows, 1 << 22):
+        p = st[r0:r0 + (1 << 22)].abs().double() ** 2
+        assert (got[r0:r0 + (1 << 22)] - p @ sign).abs().max() < 1e-5

@@ -942,6 +942,21 @@ static unsigned grid_cap(uint64_t work) {
   return b ? (unsigned)b : 1u;
 }
 
+// A launch takes 2^32 threads at most (more are cut off without an error), and
+// the kernels here use up to 512 a row and 64 a (row, term): the entry points
+// go over larger batches in slabs of rows.  2^19 rows of 96 terms are 2^31.6.
+constexpr int64_t ROW_SLAB = 1ll << 19;
+
+// f(first row, rows) for each slab until one fails
+template <class F>
+static int row_slabs(int64_t bsz, F f) {
+  for (int64_t r0 = 0; r0 < bsz; r0 += ROW_SLAB) {
+    const int rc = f(r0, bsz - r0 < ROW_SLAB ? bsz - r0 : ROW_SLAB);
+    if (rc) return rc;
+  }
+  return OK;
+}
+
 // Bytes of float workspace the expectation entry points need.
 // ---- allocation-free <Z_w> -------------------------------------------------
 // tqsv_expval_z_all_noalloc runs the same two kernels as tqsv_expval_z_all,
@@ -998,12 +1013,15 @@ TQSV_API int tqsv_expval_z_all(hipStream_t s, const void* state, int64_t bsz, in
   const int lg = ev_chunk_log2(bsz, n);
   const int64_t blocks = bsz << (n - lg);
   if (ws_bytes < blocks * (n + 1) * (int64_t)sizeof(float)) { set_error("tqsv_expval_z_all: workspace too small"); return E_ARG; }
-  k_ez_part<<<(unsigned)blocks, EV_THREADS, 0, s>>>((const float4*)state, n, lg, (float*)workspace);
-  int rc = check_launch("tqsv_expval_z_all/part");
-  if (rc) return rc;
-  const int64_t outs = bsz * n;
-  k_ez_final<<<sum_grid(outs), 256, 0, s>>>((const float*)workspace, n, 1 << (n - lg), bsz, out);
-  return check_launch("tqsv_expval_z_all/final");
+  return row_slabs(bsz, [&](int64_t r0, int64_t rows) {
+    const int lg = ev_chunk_log2(rows, n);
+    k_ez_part<<<(unsigned)(rows << (n - lg)), EV_THREADS, 0, s>>>((const float4*)((const float2*)state + (r0 << n)), n, lg,
+                                                                  (float*)workspace);
+    const int rc = check_launch("tqsv_expval_z_all/part");
+    if (rc) return rc;
+    k_ez_final<<<sum_grid(rows * n), 256, 0, s>>>((const float*)workspace, n, 1 << (n - lg), rows, out + r0 * n);
+    return check_launch("tqsv_expval_z_all/final");
+  });
 }
 
 // <Z_w> for every wire, as tqsv_expval_z_all, with no workspace argument and
@@ -1031,25 +1049,15 @@ TQSV_API int tqsv_expval_z_all_noalloc(hipStream_t s, const void* state, int64_t
   return check_launch("tqsv_expval_z_all_noalloc/final");
 }
 
-// Re <psi|P_t|psi> for nterms Pauli strings given by bit masks (in-row bit
-// positions; host arrays).  out[row * out_stride + t].
-TQSV_API int tqsv_expval_pauli(hipStream_t s, const void* state, int64_t bsz, int n, int nterms,
-                               const uint64_t* xmask, const uint64_t* zmask, float* out, int64_t out_stride,
-                               void* workspace, int64_t ws_bytes) {
-  if (!state || !out || !workspace || (nterms > 0 && (!xmask || !zmask))) {
-    set_error("tqsv_expval_pauli: null pointer");
-    return E_ARG;
-  }
-  if (bsz < 1 || n < 1 || n > 32 || nterms < 0) { set_error("tqsv_expval_pauli: need 1 <= n <= 32"); return E_ARG; }
-  if ((uintptr_t)state & 15) { set_error("tqsv_expval_pauli: state must be 16-byte aligned"); return E_ARG; }
+// The terms' values of one slab of rows.
+static int expval_pauli_rows(hipStream_t s, const void* state, int64_t bsz, int n, int nterms, const uint64_t* xmask,
+                             const uint64_t* zmask, float* out, int64_t out_stride, void* workspace,
+                             int64_t ws_bytes) {
   const int lg = ev_chunk_log2(bsz, n);
   const int64_t nchunks = 1ll << (n - lg);
   const int64_t blocks = bsz * nchunks;
   bool flips = false;
-  for (int t = 0; t < nterms; ++t) {
-    if (n < 64 && ((xmask[t] | zmask[t]) >> n)) { set_error("tqsv_expval_pauli: mask beyond n bits"); return E_ARG; }
-    flips |= xmask[t] != 0;
-  }
+  for (int t = 0; t < nterms; ++t) flips |= xmask[t] != 0;
   // terms grouped by local set, one pass per set; what fits no set, and terms
   // that all are diagonal and few, go on below
   std::vector<char> done(nterms, 0);
@@ -1116,6 +1124,25 @@ TQSV_API int tqsv_expval_pauli(hipStream_t s, const void* state, int64_t bsz, in
   return OK;
 }
 
+// Re <psi|P_t|psi> for nterms Pauli strings given by bit masks (in-row bit
+// positions; host arrays).  out[row * out_stride + t].
+TQSV_API int tqsv_expval_pauli(hipStream_t s, const void* state, int64_t bsz, int n, int nterms,
+                               const uint64_t* xmask, const uint64_t* zmask, float* out, int64_t out_stride,
+                               void* workspace, int64_t ws_bytes) {
+  if (!state || !out || !workspace || (nterms > 0 && (!xmask || !zmask))) {
+    set_error("tqsv_expval_pauli: null pointer");
+    return E_ARG;
+  }
+  if (bsz < 1 || n < 1 || n > 32 || nterms < 0) { set_error("tqsv_expval_pauli: need 1 <= n <= 32"); return E_ARG; }
+  if ((uintptr_t)state & 15) { set_error("tqsv_expval_pauli: state must be 16-byte aligned"); return E_ARG; }
+  for (int t = 0; t < nterms; ++t)
+    if ((xmask[t] | zmask[t]) >> n) { set_error("tqsv_expval_pauli: mask beyond n bits"); return E_ARG; }
+  return row_slabs(bsz, [&](int64_t r0, int64_t rows) {
+    return expval_pauli_rows(s, (const float2*)state + (r0 << n), rows, n, nterms, xmask, zmask, out + r0 * out_stride,
+                             out_stride, workspace, ws_bytes);
+  });
+}
+
 // out (+)= sum_t coef[row * coef_stride + t] P_t psi.  dotpart != null: the
 // last pass also leaves the row partials of Re <psi|out> there and sets
 // *dot_wpr to their count per row (dotpart[row * wpr + k]); 0 when the last
@@ -1178,7 +1205,10 @@ TQSV_API int tqsv_pauli_apply(hipStream_t s, void* out, const void* in, int64_t 
                               const uint64_t* xmask, const uint64_t* zmask, const void* coef, int accumulate) {
   int rc = pauli_args_ok("tqsv_pauli_apply", out, in, bsz, n, nterms, xmask, zmask, coef);
   if (rc) return rc;
-  return pauli_apply_impl(s, out, in, bsz, n, nterms, xmask, zmask, coef, nterms, accumulate, nullptr, nullptr);
+  return row_slabs(bsz, [&](int64_t r0, int64_t rows) {
+    return pauli_apply_impl(s, (float2*)out + (r0 << n), (const float2*)in + (r0 << n), rows, n, nterms, xmask, zmask,
+                            (const float2*)coef + r0 * nterms, nterms, accumulate, nullptr, nullptr);
+  });
 }
 
 // Floats of workspace tqsv_pauli_sum_grad needs (row partials of the dot).
@@ -1209,16 +1239,19 @@ TQSV_API int tqsv_pauli_sum_grad(hipStream_t s, void* out, const void* in, int64
               (long long)need);
     return E_ARG;
   }
-  int64_t wpr = 0;
-  rc = pauli_apply_impl(s, out, in, bsz, n, nterms, xmask, zmask, coef, 0, 0, workspace, &wpr);
-  if (rc) return rc;
-  if (wpr == 0) {      // the last pass computed no partials: one read of psi and out
-    const int lg = ev_chunk_log2(bsz, n);
-    k_rowdot_part<<<(unsigned)(bsz << (n - lg)), EV_THREADS, 0, s>>>((const float2*)in, (const float2*)out, n, lg,
-                                                                      workspace);
-    if ((rc = check_launch("tqsv_pauli_sum_grad/dot"))) return rc;
-    wpr = 1ll << (n - lg);
-  }
-  k_sum_chunks<<<sum_grid(bsz), 256, 0, s>>>(workspace, (int)wpr, 1, 0, bsz, 1.f, 0.f, dot, 1, 0);
-  return check_launch("tqsv_pauli_sum_grad/sum");
+  return row_slabs(bsz, [&](int64_t r0, int64_t rows) {
+    float2* o = (float2*)out + (r0 << n);
+    const float2* x = (const float2*)in + (r0 << n);
+    int64_t wpr = 0;
+    int rc = pauli_apply_impl(s, o, x, rows, n, nterms, xmask, zmask, coef, 0, 0, workspace, &wpr);
+    if (rc) return rc;
+    if (wpr == 0) {      // the last pass computed no partials: one read of psi and out
+      const int lg = ev_chunk_log2(rows, n);
+      k_rowdot_part<<<(unsigned)(rows << (n - lg)), EV_THREADS, 0, s>>>(x, o, n, lg, workspace);
+      if ((rc = check_launch("tqsv_pauli_sum_grad/dot"))) return rc;
+      wpr = 1ll << (n - lg);
+    }
+    k_sum_chunks<<<sum_grid(rows), 256, 0, s>>>(workspace, (int)wpr, 1, 0, rows, 1.f, 0.f, dot + r0, 1, 0);
+    return check_launch("tqsv_pauli_sum_grad/sum");
+  });
 }
