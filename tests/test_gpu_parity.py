@@ -658,3 +658,24 @@ def test_grouped_values_keep_their_small_digits(n, bsz):
     tol = 2.0 ** -24 * 2.0 ** (-n / 2) * (13 ** 0.5 * 6 + 6)
     assert (got - want).abs().max() < tol
     assert (total.reshape(-1) - want.sum(1)).abs().max() < tol * len(obs)
+
+
+@gpu
+@pytest.mark.parametrize("n,stage_bits,bsz", [(8, 5, 1000), (8, 5, 700), (8, 5, 1500), (10, 5, 300), (7, 4, 3000),
+                                              (12, 5, 40), (5, 5, 2500)])
+def test_partial_sums_of_every_lane_count(n, stage_bits, bsz):
+    """Rows shared by at most 2, 4, 3, 8, 2, 44 workgroups of a stage, and a workgroup of two rows: gradients of
+    the interpreting adjoint within 5e-5 of the per-gate kernels' (unit states, 30 operations whose rounding adds as
+    a random walk, observables of norm 1)."""
+    import torchquantum_amd as tq
+    rng = np.random.default_rng(80 + n)
+    ops = random_ops(n, 30, bsz, rng, names=["rx", "u3", "crx", "rzz", "cnot"])
+    grads = []
+    for mode, kw in (("fused", {"stage_bits": stage_bits, "jit": "off"}), ("pergate", {})):
+        q = _qdev(n, bsz, mode, **kw)
+        ts = apply_ops_tq(q, ops, DEV, requires_grad=True)
+        w = torch.linspace(0.5, 1.0, bsz, device=DEV)
+        (tq.expval_pauli_sum(q, ["Z" * n, "X" + "I" * (n - 1)], [0.5, 0.5]) * w).sum().backward()
+        grads.append([t.grad / max(1, bsz // t.shape[0]) for t in ts])
+    for a, b in zip(*grads):
+        assert (a - b).abs().max() < 5e-5

@@ -855,29 +855,29 @@ __global__ __launch_bounds__(512) void k_stage_adj(float2* __restrict__ psi, flo
 }
 
 // grad[row * gstride + gslot[t]] += the partials of every workgroup that
-// covered `row`, added in a fixed order: one wavefront per (row, t), lane l
-// taking the row's workgroups l, l + 64, ..., then a tree over the lanes.
+// covered `row`, added in an order fixed by the shape: 2^lg lanes per (row, t),
+// lane l taking the row's workgroups l, l + 2^lg, ..., then a tree over them.
 // Workgroup w covers groups [w * gpw, (w + 1) * gpw) and wrote its partials of
 // row r to part[(w * rpw + r - (w * gpw >> nnl)) * n_gp + t].
-// Bound by the latency of a load; with one thread walking a row's partials
-// (64 of them at 20 qubits bsz 16) that latency was paid once per partial:
-// 30.6 us per launch, 4.9 us now; 24 qubits bsz 64 (16 per row) 11.4 -> 4.9 us.
+// Bound by the latency of a load, paid once where a lane per partial takes
+// them; with more lanes than partials the idle ones take the place of other
+// values (reduce_lanes_lg).
 __global__ __launch_bounds__(256) void k_stagepart_reduce(const float* __restrict__ part, const int* __restrict__ prog,
-                                                          int64_t bsz, int64_t gpw, int64_t grid, int64_t rpw,
+                                                          int64_t bsz, int64_t gpw, int64_t grid, int64_t rpw, int lg,
                                                           float* __restrict__ grad, int64_t gstride) {
   const int n_gp = prog[H_NGP], nnl = prog[H_NNL];
   const int* __restrict__ gslot = prog + prog[H_OFF_GSLOT];
-  const int lane = threadIdx.x & 63;
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
-  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < bsz * n_gp; i += waves) {   // wave-uniform
+  const int lanes = 1 << lg, lane = threadIdx.x & (lanes - 1);
+  const int64_t step = ((int64_t)gridDim.x * blockDim.x) >> lg;
+  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> lg; i < bsz * n_gp; i += step) {
     const int64_t row = i / n_gp;
     const int t = (int)(i - row * n_gp);
     const int64_t w0 = (row << nnl) / gpw;
     int64_t w1 = (((row + 1) << nnl) - 1) / gpw;
     if (w1 > grid - 1) w1 = grid - 1;
     float s = 0.f;
-    for (int64_t w = w0 + lane; w <= w1; w += 64) s += part[(w * rpw + row - ((w * gpw) >> nnl)) * n_gp + t];
-    s = wave_sum(s);
+    for (int64_t w = w0 + lane; w <= w1; w += lanes) s += part[(w * rpw + row - ((w * gpw) >> nnl)) * n_gp + t];
+    s = wave_sum(s, lanes);
     if (lane == 0) grad[row * gstride + gslot[t]] += s;
   }
 }
@@ -1228,15 +1228,30 @@ int64_t stage_adjoint_work(const int* prog_host, int64_t gpw, int grid) {
   return (int64_t)grid * stage_rows_per_wg(prog_host, gpw) * prog_host[H_NGP];
 }
 
+// Lanes (log2) that add a row's partials: as many as the most workgroups that
+// share a row, 64 at most.  us per launch with one lane / 64 lanes for all
+// shapes / this rule: 20 qubits bsz 16 (64 partials a row) 31.8 / 5.2 / 5.0;
+// 10 qubits bsz 256 (one a row) 4.9 / 12.8 / 5.0, 8 qubits bsz 4096 5.2 / 130 /
+// 5.2, 6 qubits bsz 65536 27 / 1484 / 28.
+static int reduce_lanes_lg(int64_t groups_per_row, int64_t gpw) {
+  const int64_t per_row = groups_per_row % gpw == 0 ? groups_per_row / gpw
+                          : gpw % groups_per_row == 0 ? 1
+                                                      : groups_per_row / gpw + 2;
+  int lg = 0;
+  while (lg < 6 && (1ll << lg) < per_row) ++lg;
+  return lg;
+}
+
 // After an adjoint stage launch: add its partials into grad in a fixed order.
 int stage_adjoint_reduce(hipStream_t s, const int* prog_host, const int* prog_dev, int64_t bsz, int64_t gpw,
                          int grid, const float* work, float* grad, int64_t grad_stride) {
   const int ngp = prog_host[H_NGP];
   if (ngp == 0) return OK;
-  int64_t blocks = (bsz * ngp + 3) / 4;
+  const int lg = reduce_lanes_lg(1ll << prog_host[H_NNL], gpw);
+  int64_t blocks = (bsz * ngp + (256 >> lg) - 1) / (256 >> lg);
   if (blocks > (1ll << 20)) blocks = 1ll << 20;   // a launch takes 2^32 threads at most; the kernel strides
   k_stagepart_reduce<<<(unsigned)blocks, 256, 0, s>>>(
-      work, prog_dev, bsz, gpw, grid, stage_rows_per_wg(prog_host, gpw), grad, grad_stride);
+      work, prog_dev, bsz, gpw, grid, stage_rows_per_wg(prog_host, gpw), lg, grad, grad_stride);
   return OK;
 }
 
