@@ -206,6 +206,9 @@ int tqsv_pauli_sum_grad(tqsv_stream_t s, void* out, const void* in, int64_t bsz,
                         const uint64_t* xmask, const uint64_t* zmask, const void* coef, float* dot,
                         float* workspace, int64_t workspace_floats);
 int64_t tqsv_pauli_sum_grad_workspace_floats(int64_t bsz, int n);
+/* Passes over the state that a list of strings takes (local sets of strings,
+ * and one for each string that fits none), planned anew; host work only. */
+int tqsv_pauli_passes(int n, int nterms, const uint64_t* xmask, const uint64_t* zmask);
 
 /* ---- shot sampling: replaces measure()'s host-side random.choices over
  *      |psi|^2 (torchquantum/measurement/measurements.py:37-74), also behind

@@ -679,3 +679,32 @@ def test_partial_sums_of_every_lane_count(n, stage_bits, bsz):
         grads.append([t.grad / max(1, bsz // t.shape[0]) for t in ts])
     for a, b in zip(*grads):
         assert (a - b).abs().max() < 5e-5
+
+
+@gpu
+def test_pauli_sums_of_many_masks():
+    """600 strings of up to 6 letters on 16 wires (more different flip masks than are tried one by one) and two that
+    flip every wire: values and the sum's state gradient against the oracle, bars as in the tests above."""
+    import torchquantum_amd as tq
+    n, bsz = 16, 2
+    rng = np.random.default_rng(90)
+    strings = ["X" * n, "Y" * n]
+    while len(strings) < 602:
+        s = ["I"] * n
+        for w in rng.choice(n, rng.integers(1, 7), replace=False):
+            s[w] = "XYZ"[rng.integers(3)]
+        strings.append("".join(s))
+    coef = rng.normal(size=len(strings)) / np.sqrt(len(strings))
+    v = rng.normal(size=(bsz, 1 << n)) + 1j * rng.normal(size=(bsz, 1 << n))
+    v = (v / np.linalg.norm(v, axis=1, keepdims=True)).astype(np.complex64)
+    want = np.stack([O.expval_pauli(v.astype(np.complex128), s) for s in strings], axis=1)
+    st = torch.tensor(v, device=DEV, requires_grad=True)
+    got = tq.autograd.expval_pauli_strings(st, n, strings)
+    assert np.abs(got.detach().cpu().numpy() - want).max() < 1e-5
+    total = tq.autograd.expval_pauli_sum_state(st, n, strings, list(coef))
+    assert np.abs(total.detach().cpu().numpy() - want @ coef).max() < 1e-5
+    (a,) = torch.autograd.grad(total.sum(), st)
+    (b,) = torch.autograd.grad((got * torch.tensor(coef, dtype=torch.float32, device=DEV)).sum(), st)
+    assert (a - b).abs().max() < 1e-5
+    dot = (st.detach().conj() * a).sum(1).real.cpu().numpy() / 2
+    assert np.abs(dot - want @ coef).max() < 1e-5

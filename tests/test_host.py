@@ -795,3 +795,43 @@ def test_learned_planner_keeps_the_default_beyond_what_it_saw():
                                     (1024.0, 30, 12, 3), (None, 30, 12, 3), (256.0, 25, 0, 3)):
         pick = LearnedPlanner(Stub(max_groups)).choose_from_records(records(n, m))
         assert pick.fusion_width == width, (max_groups, n, m)
+
+
+@pytest.mark.skipif(not _native.lib_available(), reason="libtqsv.so not built")
+@pytest.mark.parametrize("n,letters", [(14, 4), (22, 4), (24, 8)])
+def test_planning_of_long_pauli_lists(n, letters):
+    """Thousands of strings: no more than 1.25 times the sets of a first fit over the list, and planned in
+    milliseconds (about 5; 0.2 s are allowed, trying every mask in every step took 0.3 s and more)."""
+    import time
+    rng = np.random.default_rng(n)
+    terms = []
+    for _ in range(8000):
+        w = rng.choice(n, rng.integers(1, letters + 1))
+        x = z = 0
+        for b in w:
+            c = rng.integers(3)
+            x |= (int(c < 2)) << int(b)
+            z |= (int(c > 0)) << int(b)
+        terms.append((x, z))
+    xs, zs = _native.u64_array([t[0] for t in terms]), _native.u64_array([t[1] for t in terms])
+    best, passes = 1e9, None
+    for _ in range(3):
+        t0 = time.perf_counter()
+        passes = _native.lib().tqsv_pauli_passes(n, len(terms), xs, zs)
+        best = min(best, time.perf_counter() - t0)
+    todo, first_fit, rest = [], 0, 0
+    for x, _ in terms:
+        if bin(x >> 4).count("1") > min(n, 13) - 4:
+            rest += 1
+        else:
+            todo.append(x >> 4)
+    while todo:
+        H, k, left = 0, 0, []
+        for h in todo:
+            if bin(H | h).count("1") <= min(n, 13) - 4 and k < 96:
+                H, k = H | h, k + 1
+            else:
+                left.append(h)
+        todo, first_fit = left, first_fit + 1
+    assert len(terms) / 96 <= passes <= 1.25 * first_fit + rest
+    assert best < 0.2, best

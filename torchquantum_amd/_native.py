@@ -55,6 +55,7 @@ SIGNATURES = {
     "tqsv_pauli_sum_grad": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_u64_p, c_u64_p,
                                     c_void_p, c_float_p, c_float_p, c_int64]),
     "tqsv_pauli_sum_grad_workspace_floats": (c_int64, [c_int64, c_int]),
+    "tqsv_pauli_passes": (c_int, [c_int, c_int, c_u64_p, c_u64_p]),
     "tqsv_batch_forward": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int]),
     "tqsv_batch_queue": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                  c_int, c_int64, c_int]),

@@ -814,50 +814,110 @@ static int pg_expval_launch(hipStream_t s, const float2* in, int n, const PGroup
 // PG_LO bits plus up to m - PG_LO higher bits that its terms flip; it is filled
 // up to m bits with the lowest unused positions (n >= 8, so m >= 8).  Terms
 // that flip more than m - PG_LO bits above PG_LO are left for the per-term
-// kernels.  A set starts from the flip mask with the most bits and grows by
-// the mask that brings in the most terms per added bit.
+// kernels.  A set starts from the flip mask with the most bits and grows:
+//   * with up to PG_EXACT different masks left, by the mask that brings in the
+//     most terms per added bit (masks x masks per step);
+//   * with more, by the bit that the most masks still lack, each weighted by
+//     8^-(bits it lacks) (masks per step).  Trying every mask for all of 8000
+//     strings of up to 4 letters on 22 wires took 0.32 s and left 90 sets,
+//     this way takes 7 ms and leaves 91; 1000 strings 3.1 and 0.5 ms, 18 sets.
+constexpr size_t PG_EXACT = 128;
+
 struct PGPlan {
   std::vector<PGroup> sets;
   std::vector<int> rest;          // terms in no set, ascending
 };
 
-static PGPlan pg_build(int n, int m, const std::vector<uint32_t>& x, const std::vector<uint32_t>& z, bool with_diag) {
+struct PGMask {
+  uint32_t bits;     // high bits flipped
+  int terms;         // terms of the list that flip them
+};
+
+// The high bits of the next set.
+static uint32_t pg_grow(const std::vector<PGMask>& masks, int room) {
+  uint32_t H = 0;
+  for (const PGMask& k : masks)
+    if (__builtin_popcount(k.bits) > __builtin_popcount(H)) H = k.bits;
+  for (;;) {
+    uint32_t best = 0;
+    if (masks.size() <= PG_EXACT) {
+      int best_gain = 0, best_bits = 1;
+      for (const PGMask& h : masks) {
+        if (!(h.bits & ~H) || __builtin_popcount(H | h.bits) > room) continue;
+        const int bits = __builtin_popcount(h.bits & ~H);
+        int gain = 0;
+        for (const PGMask& k : masks)
+          if ((k.bits & ~H) && !(k.bits & ~(H | h.bits))) gain += k.terms;
+        if (gain * best_bits > best_gain * bits) { best = h.bits; best_gain = gain; best_bits = bits; }
+      }
+    } else {
+      float weight[32] = {};
+      for (const PGMask& k : masks) {
+        const uint32_t lacks = k.bits & ~H;
+        if (!lacks || __builtin_popcount(H | k.bits) > room) continue;
+        const float w = (float)k.terms / (float)(1ull << 3 * __builtin_popcount(lacks));   // at most 9 bits
+        for (uint32_t b = lacks; b; b &= b - 1) weight[__builtin_ctz(b)] += w;
+      }
+      int top = 0;
+      for (int b = 1; b < 32; ++b)
+        if (weight[b] > weight[top]) top = b;
+      if (weight[top] > 0.f) best = 1u << top;
+    }
+    if (!best) return H;
+    H |= best;
+  }
+}
+
+static PGPlan pg_build(int n, int m, const std::vector<uint32_t>& x, const std::vector<uint32_t>& z) {
   PGPlan P;
   const int nterms = (int)x.size();
   const int room = m - PG_LO;
   const int tb = m == 13 ? 9 : 8;        // thread bits
+  const uint32_t hi_mask = ~((1u << PG_LO) - 1u);
   std::vector<int> todo;
   for (int t = 0; t < nterms; ++t) {
-    if ((x[t] || with_diag) && __builtin_popcount(x[t] >> PG_LO) <= room) todo.push_back(t);
+    if (__builtin_popcount(x[t] & hi_mask) <= room) todo.push_back(t);
     else P.rest.push_back(t);
   }
-  const uint32_t hi_mask = ~((1u << PG_LO) - 1u);
-  while (!todo.empty()) {
-    uint32_t H = 0;
-    for (int t : todo)
-      if (__builtin_popcount(x[t] & hi_mask) > __builtin_popcount(H)) H = x[t] & hi_mask;
-    for (;;) {
-      std::vector<uint32_t> open;                          // distinct masks not inside H that still fit
-      for (int t : todo) {
-        const uint32_t h = x[t] & hi_mask;
-        if ((h & ~H) && __builtin_popcount(H | h) <= room && std::find(open.begin(), open.end(), h) == open.end())
-          open.push_back(h);
+  // the different masks, in the order of their first terms
+  std::vector<PGMask> masks;
+  std::vector<int> mask_of(nterms);
+  {
+    std::vector<int> by(todo);
+    std::stable_sort(by.begin(), by.end(), [&](int p, int q) { return (x[p] & hi_mask) < (x[q] & hi_mask); });
+    std::vector<int> first(nterms, -1);        // first term of the same mask
+    for (size_t i = 0; i < by.size(); ++i)
+      first[by[i]] = i && (x[by[i]] & hi_mask) == (x[by[i - 1]] & hi_mask) ? first[by[i - 1]] : by[i];
+    for (int t : todo) {
+      if (first[t] == t) {
+        mask_of[t] = (int)masks.size();
+        masks.push_back({x[t] & hi_mask, 0});
+      } else {
+        mask_of[t] = mask_of[first[t]];
       }
-      uint32_t best = 0;
-      int best_gain = 0, best_bits = 1;
-      for (uint32_t h : open) {
-        const int bits = __builtin_popcount(h & ~H);
-        int gain = 0;
-        for (int t : todo) gain += (x[t] & hi_mask & ~H) && !(x[t] & hi_mask & ~(H | h));
-        if (gain * best_bits > best_gain * bits) { best = h; best_gain = gain; best_bits = bits; }
-      }
-      if (!best) break;
-      H |= best;
+      ++masks[mask_of[t]].terms;
     }
+  }
+  while (!todo.empty()) {
+    const uint32_t H = pg_grow(masks, room);
     std::vector<int> members, left;
     for (int t : todo) {
-      if (!(x[t] & hi_mask & ~H) && (int)members.size() < PG_MAXT) members.push_back(t);
-      else left.push_back(t);
+      if (!(x[t] & hi_mask & ~H) && (int)members.size() < PG_MAXT) {
+        members.push_back(t);
+        --masks[mask_of[t]].terms;
+      } else {
+        left.push_back(t);
+      }
+    }
+    {   // the masks that still have terms
+      std::vector<int> at(masks.size());
+      size_t kept = 0;
+      for (size_t i = 0; i < masks.size(); ++i) {
+        at[i] = (int)kept;
+        if (masks[i].terms) masks[kept++] = masks[i];
+      }
+      masks.resize(kept);
+      for (int t : left) mask_of[t] = at[mask_of[t]];
     }
     PGroup g{};
     g.m = m;
@@ -905,11 +965,9 @@ static PGPlan pg_build(int n, int m, const std::vector<uint32_t>& x, const std::
 // The sets of a list of terms, kept for the next call with the same list (a
 // loop over one observable): planning 80 terms takes about 0.1 ms.  At most
 // 64 lists; holds masks only, nothing of a state or a stream.
-static std::shared_ptr<const PGPlan> pg_plan(int n, int nterms, const uint64_t* xmask, const uint64_t* zmask,
-                                             bool with_diag) {
+static std::shared_ptr<const PGPlan> pg_plan(int n, int nterms, const uint64_t* xmask, const uint64_t* zmask) {
   struct Entry {
     int n;
-    bool with_diag;
     std::vector<uint32_t> x, z;
     std::shared_ptr<const PGPlan> plan;
   };
@@ -920,12 +978,11 @@ static std::shared_ptr<const PGPlan> pg_plan(int n, int nterms, const uint64_t* 
   {
     std::lock_guard<std::mutex> lock(mu);
     for (const Entry& e : kept)
-      if (e.n == n && e.with_diag == with_diag && e.x == x && e.z == z) return e.plan;
+      if (e.n == n && e.x == x && e.z == z) return e.plan;
   }
-  const int m = n < PG_MAXM ? n : PG_MAXM;
-  auto plan = std::make_shared<const PGPlan>(pg_build(n, m, x, z, with_diag));
+  auto plan = std::make_shared<const PGPlan>(pg_build(n, n < PG_MAXM ? n : PG_MAXM, x, z));
   std::lock_guard<std::mutex> lock(mu);
-  Entry e{n, with_diag, std::move(x), std::move(z), plan};
+  Entry e{n, std::move(x), std::move(z), plan};
   if (kept.size() < 64) kept.push_back(std::move(e));
   else kept[next++ % 64] = std::move(e);
   return plan;
@@ -1062,7 +1119,7 @@ static int expval_pauli_rows(hipStream_t s, const void* state, int64_t bsz, int 
   // that all are diagonal and few, go on below
   std::vector<char> done(nterms, 0);
   if (n >= 8 && (flips || nterms > EV_MAXT)) {
-    const std::shared_ptr<const PGPlan> P = pg_plan(n, nterms, xmask, zmask, true);
+    const std::shared_ptr<const PGPlan> P = pg_plan(n, nterms, xmask, zmask);
     for (const PGroup& g : P->sets) {
       int64_t wpr = 0;
       int rc = pg_expval_launch(s, (const float2*)state, n, g, bsz, workspace, ws_bytes, wpr);
@@ -1155,7 +1212,7 @@ static int pauli_apply_impl(hipStream_t s, void* out, const void* in, int64_t bs
   if (dot_wpr) *dot_wpr = 0;
   // terms grouped by local set: one LDS-staged pass per set
   std::shared_ptr<const PGPlan> P;
-  if (n >= 8) P = pg_plan(n, nterms, xmask, zmask, true);
+  if (n >= 8) P = pg_plan(n, nterms, xmask, zmask);
   std::vector<int> rest;
   if (P) {
     rest = P->rest;
@@ -1217,6 +1274,18 @@ TQSV_API int64_t tqsv_pauli_sum_grad_workspace_floats(int64_t bsz, int n) {
   const int64_t fused = n >= 8 ? bsz * pg_wg_per_row(bsz, n - 8, 8) : 0;       // no set has more workgroups
   const int64_t plain = bsz << (n - ev_chunk_log2(bsz, n));
   return fused > plain ? fused : plain;
+}
+
+// Passes over the state that a list of strings takes (its sets; strings that
+// fit none one each), planned anew.  Host work only.
+TQSV_API int tqsv_pauli_passes(int n, int nterms, const uint64_t* xmask, const uint64_t* zmask) {
+  if (n < 1 || n > 32 || nterms < 0 || (nterms > 0 && (!xmask || !zmask))) { set_error("tqsv_pauli_passes: bad arguments"); return E_ARG; }
+  for (int t = 0; t < nterms; ++t)
+    if ((xmask[t] | zmask[t]) >> n) { set_error("tqsv_pauli_passes: mask beyond n bits"); return E_ARG; }
+  if (n < 8) return nterms;
+  const std::vector<uint32_t> x(xmask, xmask + nterms), z(zmask, zmask + nterms);
+  const PGPlan P = pg_build(n, n < PG_MAXM ? n : PG_MAXM, x, z);
+  return (int)(P.sets.size() + P.rest.size());
 }
 
 // A Pauli sum and its state gradient in one go: out = sum_t coef[t] P_t psi
