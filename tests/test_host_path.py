@@ -122,3 +122,29 @@ def test_stale_parameters_and_pointers():
     for f in (N.host().stale, N.host().structure):
         with pytest.raises(TypeError):
             f([None])
+
+
+def test_recording_and_planning_without_the_extension(monkeypatch, tmp_path):
+    """Where nothing is built, gates and layers are recorded and plans made for the CPU as with the extension;
+    only what runs on a GPU asks for it."""
+    layers = [tq.Op1QAllLayer(op.U3, 4, has_params=True, trainable=True), tq.Op2QAllLayer(op.CNOT, 4, circular=True),
+              tq.EntanglePairwise(op.CRX, 4, has_params=True)]
+
+    def rec(q):
+        tqf.rx(q, 1, params=torch.full((1, 1), 0.3))
+        q.h(wires=2)
+        for layer in layers:
+            layer(q)
+
+    want = _outcome(rec)
+    monkeypatch.setattr(N, "HOST_PATH", tmp_path / "_tqhost.so")
+    monkeypatch.setattr(N, "_host", None)
+    assert N.host(False) is N._Unbuilt
+    assert len(want) == 13 and _outcome(rec) == want
+    q = tq.QuantumDevice(n_wires=4, device="cpu")
+    rec(q)
+    c = E.compile_tape(q._tape, 4, 1, E.EngineOptions(), "cpu")
+    assert c is E.compile_tape(list(q._tape), 4, 1, E.EngineOptions(), "cpu")
+    q._tape[0].params.add_(1)
+    with pytest.raises(RuntimeError, match="modified in place"):
+        q.flush()

@@ -116,13 +116,42 @@ def lib():
     return _lib
 
 
+HOST_PATH = Path(__file__).resolve().parent / "_tqhost.so"
 _host = None
 
 
-def host():
-    """The host extension (csrc/tqsv_host.cpp): recording, plan keys, parameter pointers."""
+class _Unbuilt:
+    """What recording and planning need of the host extension where nothing is
+    built: every gate takes the general Python path."""
+
+    @staticmethod
+    def make(*_):
+        return None
+
+    operator_op = make
+
+    @staticmethod
+    def stale(tape):
+        for i, op in enumerate(tape):
+            if op.params is not None and op.params._version != op.version:
+                return i
+        return -1
+
+    @staticmethod
+    def structure(tape):
+        return tuple((op.name, op.wires, op.inverse, op.conj, None if op.params is None else
+                      ("m", op.params.shape) if op.params.is_complex() else
+                      (op.params.shape, op.params.requires_grad, op.params.is_cuda, op.params.dtype)) for op in tape)
+
+
+def host(required: bool = True):
+    """The host extension (csrc/tqsv_host.cpp): recording, plan keys, parameter
+    pointers.  Gates are recorded and plans for the CPU made (not required)
+    without it too; whatever runs on a GPU requires it."""
     global _host
     if _host is None:
+        if not HOST_PATH.exists() and not required:
+            return _Unbuilt
         try:
             from . import _tqhost
         except ImportError as e:

@@ -85,10 +85,10 @@ class QuantumDevice(nn.Module):
                 self._sv = self._zero_state()
             return
         tape, self._tape = self._tape, []
-        i = N.host().stale(tape)
+        dev = self._sv_device()
+        i = N.host(dev.type == "cuda").stale(tape)
         if i >= 0:
             raise RuntimeError(f"parameter of gate '{tape[i].name}' was modified in place after the gate call")
-        dev = self._sv_device()
         if self._sv is None:
             dummy = torch.empty(0, dtype=C_DTYPE, device=dev)
             self._sv = run_tape(tape, dummy, self.n_wires, self.bsz, opts, init_zero=True)

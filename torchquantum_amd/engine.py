@@ -1857,7 +1857,9 @@ _plan_cache: Dict[tuple, Compiled] = {}
 
 
 def structure_key(tape: Sequence[TapeOp], n: int, bsz: int, opts: EngineOptions, device) -> tuple:
-    return (n, bsz, opts.key(), str(device), N.host().structure(tape if type(tape) is list else list(tape)))
+    where = str(device)
+    return (n, bsz, opts.key(), where,
+            N.host(where.startswith("cuda")).structure(tape if type(tape) is list else list(tape)))
 
 
 def compile_tape(tape: Sequence[TapeOp], n: int, bsz: int, opts: EngineOptions, device) -> Compiled:

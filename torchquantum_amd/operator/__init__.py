@@ -136,7 +136,7 @@ def apply_each(q_device, ops, wires):
             if spec is None:
                 spec = specs[cls] = _plain_spec(cls)
             if spec:
-                t = N.host().operator_op(op, spec, w, n)
+                t = N.host(False).operator_op(op, spec, w, n)
                 if t is not None:
                     q_device._push(t)
                     continue
