@@ -148,3 +148,31 @@ def test_recording_and_planning_without_the_extension(monkeypatch, tmp_path):
     q._tape[0].params.add_(1)
     with pytest.raises(RuntimeError, match="modified in place"):
         q.flush()
+
+
+@pytest.mark.parametrize("layer", [lambda: tq.Op1QAllLayer(op.RX, 6, has_params=True),
+                                   lambda: tq.EntanglePairwise(op.CNOT, 7)])
+def test_layers_with_too_few_ops(layer):
+    """A list shorter than the wires raises as its index does, after the gates that it has."""
+    layer, q = layer(), tq.QuantumDevice(n_wires=7, device="cpu")
+    assert len(layer.ops_all) == 6
+    del layer.ops_all[4:]
+    with pytest.raises(IndexError):
+        layer(q)
+    assert len(q._tape) == 4
+
+
+def test_layers_that_go_over_their_ops():
+    """The templates that run the ops they have do so with more and with fewer of them."""
+    ring = tq.Op2QAllLayer(op.CNOT, 5, circular=True)
+    rand = tq.RandomLayer([0, 1, 2], n_ops=6, seed=1)
+    del ring.ops_all[3:], rand.op_list[4:]
+    q = tq.QuantumDevice(n_wires=5, device="cpu")
+    ring(q)
+    assert [o.wires for o in q._tape] == [(0, 1), (1, 2), (2, 3)]
+    rand(q)
+    assert len(q._tape) == 3 + 4
+    one = tq.Op1QAllLayer(op.RX, 3, has_params=True)
+    one.ops_all.append(op.RX(has_params=True))
+    one(q)
+    assert len(q._tape) == 3 + 4 + 3

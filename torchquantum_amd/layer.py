@@ -25,7 +25,7 @@ class Op1QAllLayer(QuantumModule):
 
     @static_support
     def forward(self, q_device):
-        op.apply_each(q_device, list(self.ops_all)[:self.n_wires], range(self.n_wires))
+        op.apply_each(q_device, self.ops_all, range(self.n_wires))
 
 
 class Op2QAllLayer(QuantumModule):
@@ -142,4 +142,4 @@ class RandomLayer(QuantumModule):
 
     @static_support
     def forward(self, q_device):
-        op.apply_each(q_device, self.op_list, self.op_wires)
+        op.apply_each(q_device, self.op_list, self.op_wires[:len(self.op_list)])

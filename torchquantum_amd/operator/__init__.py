@@ -122,14 +122,18 @@ class Operator(QuantumModule):
 
 
 def apply_each(q_device, ops, wires):
-    """``op(q_device, wires=w)`` for each op and its wires, in order.  Ops of
+    """``ops[k](q_device, wires=w)`` for the k-th wires, in order.  Ops of
     this module's classes that nothing intercepts (no hooks, no tracing, no
     replaced forward, no op history) are recorded without the module call."""
     n = q_device.n_wires
     plain = not (getattr(q_device, "record_op", False) or torch._C._get_tracing_state()
                  or torch.nn.modules.module._has_any_global_hook())
     specs = {}
-    for op, w in zip(ops, wires):
+    each = iter(ops)
+    for k, w in enumerate(wires):
+        op = next(each, None)
+        if op is None:
+            op = ops[k]                   # fewer ops than wires: the list's IndexError
         if plain:
             cls = type(op)
             spec = specs.get(cls)
