@@ -176,3 +176,60 @@ def test_layers_that_go_over_their_ops():
     one.ops_all.append(op.RX(has_params=True))
     one(q)
     assert len(q._tape) == 3 + 4 + 3
+
+
+def test_replaced_module_calls_run(monkeypatch):
+    """Tracers replace nn.Module's own call and attribute look-up while they run: a layer's ops go through them."""
+    layer = tq.Op1QAllLayer(op.RY, 3, has_params=True)
+    seen = []
+    call, get = torch.nn.Module.__call__, torch.nn.Module.__getattr__
+    with monkeypatch.context() as m:
+        m.setattr(torch.nn.Module, "__call__", lambda self, *a, **k: (seen.append(self), call(self, *a, **k))[1])
+        layer(tq.QuantumDevice(n_wires=3, device="cpu"))
+    assert seen == [layer, *layer.ops_all]
+    seen.clear()
+    with monkeypatch.context() as m:
+        m.setattr(torch.nn.Module, "__getattr__", lambda self, k: (seen.append((self, k)), get(self, k))[1])
+        layer(tq.QuantumDevice(n_wires=3, device="cpu"))
+    assert [s for s in seen if s[1] == "params"] == [(o, "params") for o in layer.ops_all]
+
+
+class _Computed(op.RX):
+    params = property(lambda self: 2 * self._parameters["params"])
+
+
+class _Watched(op.RX):
+    def __getattribute__(self, k):
+        return torch.ones(1, 1) if k == "params" else super().__getattribute__(k)
+
+
+@pytest.mark.parametrize("cls", [_Computed, _Watched])
+def test_computed_parameters_are_asked_for(cls):
+    o = op.RX(has_params=True, init_params=[0.25])
+    o.__class__ = cls
+    q = tq.QuantumDevice(n_wires=2, device="cpu")
+    op.apply_each(q, [o], [1])
+    assert float(q._tape[0].params) == (0.5 if cls is _Computed else 1.0)
+
+
+@pytest.mark.parametrize("what", ["history", "global hook"])
+def test_hooks_that_turn_on_observation(what):
+    """What a hook of one op turns on applies to the ops after it in the layer."""
+    layer, q, ran, handles = tq.Op1QAllLayer(op.RY, 4, has_params=True), tq.QuantumDevice(n_wires=4, device="cpu"), [], []
+
+    def hook(m, i):
+        if what == "history":
+            q.record_op = True
+        else:
+            handles.append(torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: ran.append(m)))
+
+    layer.ops_all[1].register_forward_pre_hook(hook)
+    try:
+        layer(q)
+    finally:
+        for h in handles:
+            h.remove()
+    if what == "history":
+        assert [h["wires"] for h in q.op_history] == [1, 2, 3]
+    else:
+        assert [m for m in ran if isinstance(m, op.RY)][-2:] == list(layer.ops_all)[2:]

@@ -124,10 +124,10 @@ class Operator(QuantumModule):
 def apply_each(q_device, ops, wires):
     """``ops[k](q_device, wires=w)`` for the k-th wires, in order.  Ops of
     this module's classes that nothing intercepts (no hooks, no tracing, no
-    replaced forward, no op history) are recorded without the module call."""
+    replaced call or forward, no op history) are recorded without the module
+    call."""
     n = q_device.n_wires
-    plain = not (getattr(q_device, "record_op", False) or torch._C._get_tracing_state()
-                 or torch.nn.modules.module._has_any_global_hook())
+    plain = _unobserved(q_device)
     specs = {}
     each = iter(ops)
     for k, w in enumerate(wires):
@@ -145,12 +145,26 @@ def apply_each(q_device, ops, wires):
                     q_device._push(t)
                     continue
         op(q_device, wires=w)
+        plain = _unobserved(q_device)     # a hook of that call may have changed it
+
+
+def _unobserved(q_device) -> bool:
+    """No op history, tracing or hook of all modules sees the calls of ops."""
+    return not (getattr(q_device, "record_op", False) or torch._C._get_tracing_state()
+                or torch.nn.modules.module._has_any_global_hook())
+
+
+# what a module call is made of, as found at import: tracers replace these on
+# nn.Module itself for as long as they run
+_MODULE_PARTS = ("__call__", "__getattr__", "__setattr__", "__getattribute__")
+_MODULE_CALL = tuple(getattr(nn.Module, a) for a in _MODULE_PARTS)
+_OPERATOR_FORWARD = Operator.forward
 
 
 def _plain_spec(cls):
     """(gate, wires, parameters) of a class whose call only records that gate, else ()."""
-    if not issubclass(cls, Operator) or cls.forward is not Operator.forward or cls.__call__ is not nn.Module.__call__ \
-            or cls.__getattr__ is not nn.Module.__getattr__ or cls.__setattr__ is not nn.Module.__setattr__:
+    if not issubclass(cls, Operator) or cls.forward is not _OPERATOR_FORWARD or hasattr(cls, "params") \
+            or any(getattr(cls, a) is not f for a, f in zip(_MODULE_PARTS, _MODULE_CALL)):
         return ()
     return getattr(cls.func, "plain_spec", None) or ()
 
