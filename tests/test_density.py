@@ -243,3 +243,41 @@ def test_density_compiled_stages():
     ref = OD.run_density_ops(seq, n, bsz)
     assert np.abs(out["on"] - out["off"]).max() < 1e-6
     assert np.abs(out["on"] - ref).max() < 1e-5
+
+
+def _random_density(n, bsz, seed):
+    rng = np.random.default_rng(seed)
+    a = rng.normal(size=(bsz, 1 << n, 1 << n)) + 1j * rng.normal(size=(bsz, 1 << n, 1 << n))
+    rho = a @ np.conj(np.swapaxes(a, 1, 2))
+    return rho / np.trace(rho, axis1=1, axis2=2)[:, None, None]
+
+
+@pytest.mark.parametrize("budget,small,ring", [(1 << 24, 1 << 16, 1 << 18), (5 * 16 * 7, 1 << 16, 1 << 18),
+                                               (5 * 16 * 7, 64, 64), (1, 1 << 16, 1 << 18)])
+def test_density_values_within_the_gather_budget(monkeypatch, budget, small, ring):
+    """30 strings of 5 rows in one gather, in several and one by one; no gather is larger than the budget over all
+    rows (or one string's), kept and fresh tables agree.  complex64 sums over 16 entries of size <= 1: 1e-6."""
+    import torchquantum_amd as tq
+    from torchquantum_amd import noisedevice as ND
+    n, bsz = 4, 5
+    rho = _random_density(n, bsz, 3)
+    dev = tq.NoiseDevice(n_wires=n, bsz=bsz, device="cpu")
+    dev.densities = torch.tensor(rho, dtype=torch.complex64).reshape([bsz] + [2] * (2 * n))
+    rng = np.random.default_rng(4)
+    strings = ["".join(rng.choice(list("IXYZ"), n)) for _ in range(30)]
+    sizes = []
+    upload, copied = ND.E.upload, ND._copied
+    monkeypatch.setattr(ND.E, "upload", lambda h, d: (sizes.append(h.size if h.dtype == np.int64 else 0), upload(h, d))[1])
+    monkeypatch.setattr(ND, "_copied", lambda h, d: (sizes.append(h.size if h.dtype == np.int64 else 0), copied(h, d))[1])
+    monkeypatch.setattr(ND, "CHUNK", budget)
+    monkeypatch.setattr(ND, "SMALL_TABLE", small)
+    monkeypatch.setattr(ND, "RING_TABLE", ring)
+    want = np.stack([OD.expval_pauli(rho, s) for s in strings], axis=1)
+    for again in range(2):
+        got = ND.density_expval_strings(dev, strings if again else iter(strings))
+        assert got.shape == (bsz, 30)
+        assert np.abs(got.numpy() - want).max() < 1e-6
+    assert sum(sizes) == 2 * 30 << n
+    assert max(sizes) * bsz <= max(budget, bsz << n)
+    with pytest.raises(RuntimeError):
+        ND.density_expval_strings(dev, [])

@@ -250,7 +250,8 @@ def _string_tables(n: int, observables: Sequence[str]):
 
 _small_tables = functools.lru_cache(maxsize=32)(_string_tables)
 SMALL_TABLE = 1 << 16          # entries of a table that is kept for the next call with the same strings
-CHUNK = 1 << 22                # entries gathered per row at a time
+RING_TABLE = 1 << 18           # entries of a table that goes through the pinned upload buffers, which stay allocated
+CHUNK = 1 << 24                # entries gathered at a time over all rows (128 MiB, and their products as much)
 
 
 def density_expval_strings(dev: NoiseDevice, observables: Sequence[str]) -> torch.Tensor:
@@ -263,12 +264,20 @@ def density_expval_strings(dev: NoiseDevice, observables: Sequence[str]) -> torc
     n = dev.n_wires
     flat = dev.reg.get_states_1d()                         # [bsz, 4^n]
     d = 1 << n
+    observables = list(observables)
+    if not observables:
+        raise RuntimeError("no observables")
     cols = []
-    per = max(1, CHUNK >> n)
+    per = max(1, CHUNK // (flat.shape[0] << n))
     for t0 in range(0, len(observables), per):
         obs = tuple(observables[t0:t0 + per])
         idx, sgn, re, im = (_small_tables if len(obs) * d <= SMALL_TABLE else _string_tables)(n, obs)
-        g = flat[:, E.upload(idx.reshape(-1), flat.device)].reshape(-1, len(obs), d)
-        s = (g * E.upload(sgn, flat.device)).sum(-1)           # sum_r sign rho[r, r^x]
+        put = E.upload if len(obs) * d <= RING_TABLE else _copied
+        g = flat[:, put(idx.reshape(-1), flat.device)].reshape(-1, len(obs), d)
+        s = (g * put(sgn, flat.device)).sum(-1)                # sum_r sign rho[r, r^x]
         cols.append(s.real * E.upload(re, flat.device) - s.imag * E.upload(im, flat.device))    # Re(i^ny s)
     return torch.cat(cols, dim=-1)
+
+
+def _copied(host: np.ndarray, device: torch.device) -> torch.Tensor:
+    return torch.from_numpy(host).to(device)
