@@ -903,6 +903,17 @@ struct BatchItem {
 // are what another loads.  With plain accesses every item ended with an L2
 // write-back and every wait with an invalidation, which the other workgroups
 // of the XCD paid for too (64 circuits: 7.46 -> 7.14 ms).
+//
+// One workgroup's stores are ordered before another's loads by the hardware,
+// not by the language's release and acquire (which would be those cache
+// operations): on gfx950 agent-scope accesses are sc1 loads and stores, an sc1
+// store is acknowledged once it is where every XCD's sc1 loads look, and
+// vmcnt counts it until then.  So every access to the state inside
+// batch_item<true> has to be a state_load or state_store -- a plain load could
+// read a stale L2 line -- and a wave publishes only after s_waitcnt vmcnt(0).
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "k_batch_queue relies on gfx950's sc1 accesses and vmcnt"
+#endif
 template <bool COHERENT>
 __device__ __forceinline__ float2 state_load(const float2* p) {
   if constexpr (COHERENT) {
