@@ -673,7 +673,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       __syncthreads();
     }
     float2 an[NR];
-    {
+    {   // the last group once more at the end, from cache: guarded, 1 group per workgroup gains 3% (22 qubits bsz 1 with
+        // 60 strings 122 -> 118 us) and 16 of them lose 3% (24 qubits bsz 4 680 -> 701 us)
       const uint64_t gn = (uint64_t)(grp + 1 < g0 + gpw ? grp + 1 : grp);
       pg_load<NR, BIG>(in + ((gn >> g.nnl) << n) + pg_group_offset(g, gn & rmask), tsc, rsc, an);
     }
@@ -761,7 +762,8 @@ static int64_t pg_wg_per_row(int64_t bsz, int nnl, int m) {
 
 // f with the threads and slots of a set's width -- m = 8 + log2(NR) with 256
 // threads up to 12 bits, 512 threads for 13 -- and whether buffer
-// instructions do not reach its positions.
+// instructions do not reach its positions.  (Below 13 bits a set is the whole
+// row of m wires.)
 template <class F>
 static int pg_dispatch(const PGroup& g, F f) {
   using std::integral_constant;
@@ -770,14 +772,13 @@ static int pg_dispatch(const PGroup& g, F f) {
   const integral_constant<int, 16> n16;
   const std::false_type buf;
   const std::true_type big;
-  const bool far = g.lpos[g.m - 1] > 27;
   switch (g.m) {
     case 8: return f(t256, integral_constant<int, 1>(), buf);
     case 9: return f(t256, integral_constant<int, 2>(), buf);
     case 10: return f(t256, integral_constant<int, 4>(), buf);
     case 11: return f(t256, integral_constant<int, 8>(), buf);
-    case 12: return far ? f(t256, n16, big) : f(t256, n16, buf);
-    default: return far ? f(t512, n16, big) : f(t512, n16, buf);
+    case 12: return f(t256, n16, buf);
+    default: return g.lpos[g.m - 1] > 27 ? f(t512, n16, big) : f(t512, n16, buf);
   }
 }
 
