@@ -109,8 +109,9 @@ class Autotuner:
 
 class LearnedPlanner:
     """Pick the candidate with the smallest predicted time (no launches).
-    For a circuit whose stages fill the chip, when no timed one's did, the
-    first candidate is taken (MLPCostModel.covers)."""
+    Where the model learned from no plan that fills the chip, a circuit with
+    more groups per stage than any it learned from takes the first candidate
+    (MLPCostModel.covers)."""
 
     def __init__(self, model: MLPCostModel, candidates: Sequence[E.EngineOptions] = DEFAULT_CANDIDATES):
         self.model = model

@@ -156,14 +156,17 @@ class MLPCostModel:
     def groups(X: np.ndarray) -> np.ndarray:
         """Workgroup-sized pieces a stage of each plan has to work on."""
         X = np.atleast_2d(np.asarray(X, dtype=np.float64))
-        return np.where(X[:, 14] > 0, np.exp2(X[:, 0] - X[:, 14]), 1.0)
+        amps, bits = X[:, FEATURES.index("log2_amps")], X[:, FEATURES.index("stage_bits")]
+        return np.where(bits > 0, np.exp2(amps - bits), 1.0)
 
     def covers(self, X: np.ndarray) -> bool:
-        """Whether the timings the model learned from say something about
-        plans of this size.  Up to one group per CU an operation costs its
+        """Whether the model's choice is taken for plans of this size: always
+        if it learned from plans of more than one group per CU, else up to the
+        largest it learned from.  Up to one group per CU an operation costs its
         latency, beyond that its arithmetic, and plans rank differently:
         with circuits of at most 20 qubits timed (256 groups, fusion width 2
-        ahead by 3-13%), width 2 was 8-10% slower than width 1 at 21 and 22."""
+        ahead by 3-13%), width 2 was 8-10% slower than width 1 at 21 and 22.
+        Chosen on those circuits; other candidates or sizes may rank otherwise."""
         return self.max_groups is None or self.max_groups > CUS or float(self.groups(X).max()) <= self.max_groups
 
     @staticmethod
