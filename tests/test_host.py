@@ -725,6 +725,31 @@ def test_batch_queue_order():
         assert q["b"]["state_off"][k] == cb.state_off[c]
 
 
+@pytest.mark.skipif(not _native.lib_available(), reason="libtqsv.so not built")
+@pytest.mark.parametrize("n_circ,n_range", [(1, (4, 5)), (3, (16, 17)), (20, (5, 18)), (40, (17, 18)), (30, (18, 19))])
+def test_batch_items_cover_every_group_once(n_circ, n_range):
+    """Work items sized by the batch: every stage's groups in order, each once, items of 1 to 6 groups and at least
+    4 of them where a circuit's widest stage has that many groups; a size given by the caller stands."""
+    from torchquantum_amd import batch as B
+    circs = B.random_circuits(n_circ=n_circ, n_range=n_range, depth_range=(2, 4), seed=n_circ)
+    for given in (None, 3):
+        cb = B.CircuitBatch(circs, device="cpu", groups_per_item=given)
+        per = cb._groups_per_item()
+        q = np.frombuffer(cb.queue.numpy().tobytes(), dtype=B.QUEUE_ITEM)
+        for i in range(n_circ):
+            widest = max(1 << (cb.ns[i] - m) for m in cb.stage_m[i])
+            assert 1 <= per[i] <= 6 and (widest < 4 or -(-widest // per[i]) >= 4)
+            for prog, m in zip(cb.stage_offsets[i], cb.stage_m[i]):
+                mine = q["b"][(q["circ"] == i) & (q["b"]["prog_off"] == prog)]
+                edges = np.append(mine["g0"], mine["g1"][-1])
+                step = per[i] if given is None else given
+                assert np.array_equal(mine["g1"], edges[1:]) and edges[0] == 0 and edges[-1] == 1 << (cb.ns[i] - m)
+                assert (np.diff(edges) <= step).all() and (np.diff(edges)[:-1] == step).all()
+    # a mean level of some 1536 items: several groups per item where there are 1.5 times as many groups
+    level = sum(1 << (n - m) for n, ms in zip(cb.ns, cb.stage_m) for m in ms) / max(len(ms) for ms in cb.stage_m)
+    assert (max(per) > 1) == (level > 1.5 * 1536)
+
+
 def test_default_stage_width_follows_state_size():
     """Automatic stage width: 13 local bits for states of more than 512 MiB
     (HBM-resident: fewer passes win), 12 below (cache-resident), never more
