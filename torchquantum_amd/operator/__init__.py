@@ -129,11 +129,7 @@ def apply_each(q_device, ops, wires):
     n = q_device.n_wires
     plain = _unobserved(q_device)
     specs = {}
-    each = iter(ops)
-    for k, w in enumerate(wires):
-        op = next(each, None)
-        if op is None:
-            op = ops[k]                   # fewer ops than wires: the list's IndexError
+    for op, w in zip(ops, wires):
         if plain:
             cls = type(op)
             spec = specs.get(cls)
@@ -146,6 +142,8 @@ def apply_each(q_device, ops, wires):
                     continue
         op(q_device, wires=w)
         plain = _unobserved(q_device)     # a hook of that call may have changed it
+    if len(ops) < len(wires):
+        ops[len(ops)]                     # the list's IndexError
 
 
 def _unobserved(q_device) -> bool:
@@ -156,15 +154,15 @@ def _unobserved(q_device) -> bool:
 
 # what a module call is made of, as found at import: tracers replace these on
 # nn.Module itself for as long as they run
-_MODULE_PARTS = ("__call__", "__getattr__", "__setattr__", "__getattribute__")
-_MODULE_CALL = tuple(getattr(nn.Module, a) for a in _MODULE_PARTS)
-_OPERATOR_FORWARD = Operator.forward
+_CALL, _GETATTR, _SETATTR = nn.Module.__call__, nn.Module.__getattr__, nn.Module.__setattr__
+_GETATTRIBUTE, _FORWARD = nn.Module.__getattribute__, Operator.forward
 
 
 def _plain_spec(cls):
     """(gate, wires, parameters) of a class whose call only records that gate, else ()."""
-    if not issubclass(cls, Operator) or cls.forward is not _OPERATOR_FORWARD or hasattr(cls, "params") \
-            or any(getattr(cls, a) is not f for a, f in zip(_MODULE_PARTS, _MODULE_CALL)):
+    if not issubclass(cls, Operator) or cls.forward is not _FORWARD or cls.__call__ is not _CALL \
+            or cls.__getattr__ is not _GETATTR or cls.__setattr__ is not _SETATTR \
+            or cls.__getattribute__ is not _GETATTRIBUTE or hasattr(cls, "params"):
         return ()
     return getattr(cls.func, "plain_spec", None) or ()
 
