@@ -73,6 +73,26 @@ def test_captured_circuit(mode, n, rows):
 
 
 @gpu
+def test_captured_circuit_without_matrices():
+    st = torch.randn(3, 32, dtype=torch.complex64, device=DEV)
+
+    def run():
+        q = tq.QuantumDevice(n_wires=5, bsz=3, device=DEV)
+        q.set_states(st)
+        tqf.swap(q, [0, 3])
+        tqf.swap(q, [1, 4])
+        return q.get_states_1d()
+
+    g, out = _capture(run)
+    for k in range(3):
+        st.copy_(torch.randn(3, 32, dtype=torch.complex64, device=DEV))
+        _other_work(k)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, run())
+
+
+@gpu
 def test_pauli_sums_of_a_given_state_are_refused():
     """Coefficients and index tables come from host memory: their copies are refused while a graph is recorded, as
     torch refuses a copy from pageable memory, and work after the recording as before."""

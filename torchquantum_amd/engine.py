@@ -727,10 +727,19 @@ def _check_dev_layout():
 
 def _capturing(device: torch.device) -> bool:
     """Whether the device's current stream is recording a graph."""
-    if device.index is None or device.index == torch.cuda.current_device():
-        return torch.cuda.is_current_stream_capturing()
+    if device.index is None or device.index == torch._C._cuda_getDevice():
+        return torch._C._cuda_isCurrentStreamCapturing()
     with torch.cuda.device(device):
-        return torch.cuda.is_current_stream_capturing()
+        return torch._C._cuda_isCurrentStreamCapturing()
+
+
+def _staged(host: np.ndarray, device: torch.device) -> torch.Tensor:
+    if device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    ring = _RINGS.get(device)
+    if ring is None:
+        ring = _RINGS.setdefault(device, _PinnedRing())
+    return ring.upload(host, device)
 
 
 def upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
@@ -743,12 +752,7 @@ def upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
         return torch.from_numpy(host).to(device)
     if _capturing(device):
         raise RuntimeError("a copy from a shared host buffer cannot be captured into a graph")
-    if device.index is None:
-        device = torch.device("cuda", torch.cuda.current_device())
-    ring = _RINGS.get(device)
-    if ring is None:
-        ring = _RINGS.setdefault(device, _PinnedRing())
-    return ring.upload(host, device)
+    return _staged(host, device)
 
 
 def put(host: np.ndarray, device: torch.device) -> torch.Tensor:
@@ -1677,7 +1681,9 @@ class Compiled:
         if torch.device(self.device).type != "cuda":
             return torch.from_numpy(host).to(self.device)
         device = torch.device(self.device)
-        pool = (put if _capturing(device) else upload)(host, device)
+        if host.size == 0:
+            return torch.empty(0, dtype=torch.complex64, device=device)
+        pool = (put if _capturing(device) else _staged)(host, device)
         if len(self.dev_ops):
             _check_dev_layout()
             base = pool.data_ptr() + 8 * self.pool_len
