@@ -844,16 +844,14 @@ def test_planning_of_long_pauli_lists(n, letters):
         t0 = time.perf_counter()
         passes = _native.lib().tqsv_pauli_passes(n, len(terms), xs, zs)
         best = min(best, time.perf_counter() - t0)
-    todo, first_fit, rest = [], 0, 0
-    for x, _ in terms:
-        if bin(x >> 4).count("1") > min(n, 13) - 4:
-            rest += 1
-        else:
-            todo.append(x >> 4)
+    ones = bytes(bin(v).count("1") for v in range(1 << (n - 4)))
+    room = min(n, 13) - 4
+    todo = [x >> 4 for x, _ in terms if ones[x >> 4] <= room]
+    first_fit, rest = 0, len(terms) - len(todo)
     while todo:
         H, k, left = 0, 0, []
         for h in todo:
-            if bin(H | h).count("1") <= min(n, 13) - 4 and k < 96:
+            if k < 96 and ones[H | h] <= room:
                 H, k = H | h, k + 1
             else:
                 left.append(h)
