@@ -128,9 +128,9 @@ __device__ __forceinline__ uint64_t insert_zeros(uint64_t i, const InsertSpec& s
   return i;
 }
 
-// Sum over the first `width` lanes of a wavefront (width: power of two <= 64;
-// smaller than 64 only for workgroups narrower than one wavefront, whose
-// upper lanes do not exist).  Lane 0 holds the total.
+// Sum over the lanes of each aligned run of `width` lanes of a wavefront
+// (width: power of two <= 64; in workgroups narrower than one wavefront the
+// upper lanes do not exist), in every lane of the run.
 __device__ __forceinline__ float wave_sum(float v, int width = 64) {
   for (int o = width >> 1; o >= 1; o >>= 1) v += __shfl_xor(v, o, width);
   return v;
