@@ -5,12 +5,15 @@ the current contents of the parameter tensors it reads), whatever the program
 has run on the device since: each replay is compared with an eager run of the
 same circuit, and eager work of other circuits lies between them.
 """
+import gc
+
 import numpy as np
 import pytest
 import torch
 
 import torchquantum_amd as tq
 import torchquantum_amd.functional as tqf
+from torchquantum_amd import engine as E
 
 gpu = pytest.mark.gpu
 DEV = "cuda"
@@ -63,6 +66,8 @@ def test_captured_circuit(mode, n, rows):
 
     g, out = _capture(run)
     for k in range(4):
+        E._plan_cache.clear()            # as after many other circuits: the graph's plan has to outlive the cache
+        gc.collect()
         theta.fill_(0.3 + k)
         _other_work(k)
         g.replay()
@@ -85,6 +90,8 @@ def test_captured_circuit_without_matrices():
 
     g, out = _capture(run)
     for k in range(3):
+        E._plan_cache.clear()
+        gc.collect()
         st.copy_(torch.randn(3, 32, dtype=torch.complex64, device=DEV))
         _other_work(k)
         g.replay()

@@ -1681,9 +1681,12 @@ class Compiled:
         if torch.device(self.device).type != "cuda":
             return torch.from_numpy(host).to(self.device)
         device = torch.device(self.device)
+        capturing = _capturing(device)
+        if capturing:
+            _CAPTURED.add(self)
         if host.size == 0:
             return torch.empty(0, dtype=torch.complex64, device=device)
-        pool = (put if _capturing(device) else _staged)(host, device)
+        pool = (put if capturing else _staged)(host, device)
         if len(self.dev_ops):
             _check_dev_layout()
             base = pool.data_ptr() + 8 * self.pool_len
@@ -1860,6 +1863,9 @@ def _member_slots(op: TapeOp):
 
 _cache_lock = threading.Lock()
 _plan_cache: Dict[tuple, Compiled] = {}
+# plans that a graph was recorded with: its replays read their programs on the
+# device, so they outlive the cache (one per circuit structure recorded)
+_CAPTURED: set = set()
 
 
 def structure_key(tape: Sequence[TapeOp], n: int, bsz: int, opts: EngineOptions, device) -> tuple:
