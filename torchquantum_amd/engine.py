@@ -1676,7 +1676,8 @@ class Compiled:
     # ---------------------------------------------------------------- values
     def pool(self, tape: Sequence[TapeOp], with_grad: bool, with_adj: bool) -> torch.Tensor:
         """The matrix pool on the device: staged through pinned host memory and
-        copied asynchronously on the current stream (no wait for queued work)."""
+        copied asynchronously on the current stream (no wait for queued work),
+        or, while the stream is recorded into a graph, as part of the graph."""
         host = self.pool_host(tape, with_grad, with_adj)
         if torch.device(self.device).type != "cuda":
             return torch.from_numpy(host).to(self.device)
