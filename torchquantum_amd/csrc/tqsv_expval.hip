@@ -418,24 +418,27 @@ __device__ __forceinline__ float flip_sign(float v, uint32_t neg) {   // neg: 0 
 
 // Bit 31 - (t & 31) of word t >> 5: the sign a term has for thread-field tid
 // (its parity under the term's thread mask).  The same for every group, and
-// walked by shifting left as the terms go by.
-constexpr int PG_WORDS = (PG_MAXT + 31) / 32;
+// walked by shifting left as the terms go by.  Three scalars, not an array:
+// an array indexed by a word number goes to LDS, at an address for which every
+// wavefront reads the dispatch packet in host memory (14 us a launch: one
+// string, 20 qubits bsz 3: 27.2 us, 18.9 without; 8 qubits bsz 500: 17.5, 4.2).
+static_assert(PG_MAXT == 96, "three words of signs");
+struct LaneSigns {
+  uint32_t a, b, c;
+};
 
-__device__ __forceinline__ void pg_lane_signs(const PGroup& g, uint32_t tid, uint32_t (&lw)[PG_WORDS]) {
-#pragma unroll
-  for (int k = 0; k < PG_WORDS; ++k) {
-    uint32_t w = 0;
-    for (int t = 32 * k; t < g.nt && t < 32 * k + 32; ++t) w |= (__popc(tid & g.zt[t]) & 1u) << (31 - (t & 31));
-    lw[k] = w;
-  }
+__device__ __forceinline__ uint32_t pg_lane_word(const PGroup& g, uint32_t tid, int first) {
+  uint32_t w = 0;
+  for (int t = first; t < g.nt && t < first + 32; ++t) w |= (__popc(tid & g.zt[t]) & 1u) << (31 - (t & 31));
+  return w;
 }
 
-__device__ __forceinline__ uint32_t pg_word(const uint32_t (&lw)[PG_WORDS], int k) {   // k wave-uniform
-  uint32_t w = lw[0];
-#pragma unroll
-  for (int i = 1; i < PG_WORDS; ++i)
-    if (k == i) w = lw[i];
-  return w;
+__device__ __forceinline__ LaneSigns pg_lane_signs(const PGroup& g, uint32_t tid) {
+  return {pg_lane_word(g, tid, 0), pg_lane_word(g, tid, 32), pg_lane_word(g, tid, 64)};
+}
+
+__device__ __forceinline__ uint32_t pg_word(const LaneSigns& s, int k) {   // k wave-uniform
+  return k == 0 ? s.a : k == 1 ? s.b : s.c;
 }
 
 // acc[r] += (+-c) v_r, or (+-i c) v_r with IM, the sign from bit r of pm with
@@ -540,8 +543,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // this thread's own term, whose coefficient it puts into cg, and its signs of all terms
   const uint32_t my_zg = tid < g.nt ? g.zg[tid] : 0u;
   const int my_col = tid < g.nt ? g.col[tid] : 0;
-  uint32_t lw[PG_WORDS];
-  pg_lane_signs(g, (uint32_t)tid | 0x10000u, lw);
+  const LaneSigns lw = pg_lane_signs(g, (uint32_t)tid | 0x10000u);
   const int64_t g0 = (int64_t)blockIdx.x * gpw;
   const int64_t g1 = g0 + gpw < n_groups ? g0 + gpw : n_groups;
   const uint64_t rmask = (1ull << g.nnl) - 1ull;
@@ -573,7 +575,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       const uint64_t gn = (uint64_t)grp + 1;
       pg_load<NR, BIG>(in + ((gn >> g.nnl) << n) + pg_group_offset(g, gn & rmask), tsc, rsc, a);
     }
-    uint32_t w = lw[0];
+    uint32_t w = lw.a;
     uint32_t x = g.ex[0], pm = g.epm[0];
     int t = 0, tend = g.ebeg[1];
     for (int e = 0; e < g.ne; ++e) {
@@ -657,8 +659,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   for (int r = 0; r < NR; ++r) rsc[r] = pg_scatter(g, (uint32_t)r * NT);
   for (int t = tid; t < (NT / 64) * PG_MAXT; t += NT) gacc[0][t] = 0.0;
   if (tid < g.nt) zgs[tid] = g.zg[tid];
-  uint32_t lw[PG_WORDS];
-  pg_lane_signs(g, (uint32_t)tid, lw);
+  const LaneSigns lw = pg_lane_signs(g, (uint32_t)tid);
   const int64_t g0 = (int64_t)blockIdx.x * gpw;
   const uint64_t rmask = (1ull << g.nnl) - 1ull;
   const char* b8 = (const char*)buf;
