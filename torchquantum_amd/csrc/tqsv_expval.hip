@@ -657,7 +657,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // term before).
 // part[(blockIdx.x * nt + t) * 2] = the partial of term t, and what float32
 // leaves off it.
-template <int NT, int NR, bool BIG>
+// ONE: one group per workgroup (gpw 1), so nothing is loaded ahead (22 qubits
+// bsz 1 with 60 strings 77 -> 70 us, 20 qubits bsz 4 with 40 45 -> 42 us).
+template <int NT, int NR, bool BIG, bool ONE>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_pauli_group_expval(const float2* __restrict__ in, int n, PGroup g,
                                                            int64_t gpw, float* __restrict__ part) {
   __shared__ float2 buf[NR * NT];
@@ -687,8 +689,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       __syncthreads();
     }
     float2 an[NR];
-    {   // the last group once more at the end, from cache: guarded, 1 group per workgroup gains 3% (22 qubits bsz 1 with
-        // 60 strings 122 -> 118 us) and 16 of them lose 3% (24 qubits bsz 4 680 -> 701 us)
+    if constexpr (!ONE) {   // the last group once more at the end: behind a branch 24 qubits bsz 4 took 671 instead of 655 us
       const uint64_t gn = (uint64_t)(grp + 1 < g0 + gpw ? grp + 1 : grp);
       pg_load<NR, BIG>(in + ((gn >> g.nnl) << n) + pg_group_offset(g, gn & rmask), tsc, rsc, an);
     }
@@ -721,8 +722,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       const int t = t0 + (lane >> 3);
       if ((lane & 7) == 0 && t < g.nt) wacc[t] += (__popc(goff & zgs[t]) & 1u) ? -c : c;
     }
+    if constexpr (!ONE) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r) a[r] = an[r];
+      for (int r = 0; r < NR; ++r) a[r] = an[r];
+    }
   }
   __syncthreads();
   for (int t = tid; t < g.nt; t += NT) {
@@ -820,7 +823,15 @@ static int pg_expval_launch(hipStream_t s, const float2* in, int n, const PGroup
   const int64_t grid = bsz * wpr;
   if (grid > 0x7fffffffll || ws_bytes < grid * 2 * g.nt * (int64_t)sizeof(float)) return 1;   // caller falls back
   return pg_dispatch(g, [&](auto nt, auto nr, auto big) {
-    k_pauli_group_expval<nt(), nr(), big()><<<(unsigned)grid, nt(), 0, s>>>(in, n, g, gpw, (float*)ws);
+    auto launch = [&](auto one) {
+      k_pauli_group_expval<nt(), nr(), big(), one()><<<(unsigned)grid, nt(), 0, s>>>(in, n, g, gpw, (float*)ws);
+    };
+    if constexpr (decltype(nt)::value == 512) {      // narrower sets are whole rows: one group
+      if (gpw > 1) launch(std::false_type());
+      else launch(std::true_type());
+    } else {
+      launch(std::true_type());
+    }
     return check_launch("tqsv_expval_pauli/group");
   });
 }
