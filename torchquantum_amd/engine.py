@@ -1685,9 +1685,9 @@ class Compiled:
         copied asynchronously on the current stream (no wait for queued work),
         or, while the stream is recorded into a graph, as part of the graph."""
         host = self.pool_host(tape, with_grad, with_adj)
-        if torch.device(self.device).type != "cuda":
-            return torch.from_numpy(host).to(self.device)
         device = torch.device(self.device)
+        if device.type != "cuda":
+            return torch.from_numpy(host).to(device)
         capturing = _capturing(device)
         if capturing:
             _CAPTURED.add(self)

@@ -130,7 +130,7 @@ def _make_gate(name: str):
         # the plain form (a fixed-width gate on int wires, no parameter or a
         # real [rows, P] tensor, no op history) is recorded natively
         if plain and comp_method == "bmm" and not getattr(q_device, "record_op", False):
-            op = N.host(False).make(cname, nw, npar, wires, params, inverse, q_device.n_wires)
+            op = (N._host or N.host(False)).make(cname, nw, npar, wires, params, inverse, q_device.n_wires)
             if op is not None:
                 q_device._push(op)
                 return

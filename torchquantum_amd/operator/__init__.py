@@ -129,6 +129,7 @@ def apply_each(q_device, ops, wires):
     n = q_device.n_wires
     plain = _unobserved(q_device)
     specs = {}
+    host = N.host(False)
     for op, w in zip(ops, wires):
         if plain:
             cls = type(op)
@@ -136,7 +137,7 @@ def apply_each(q_device, ops, wires):
             if spec is None:
                 spec = specs[cls] = _plain_spec(cls)
             if spec:
-                t = N.host(False).operator_op(op, spec, w, n)
+                t = host.operator_op(op, spec, w, n)
                 if t is not None:
                     q_device._push(t)
                     continue
