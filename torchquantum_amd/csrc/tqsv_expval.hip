@@ -532,7 +532,8 @@ __device__ __forceinline__ double pg_sum8(const float (&v)[8], int lane) {
 // of 6 and 6, chosen by what they bring in: 22 qubits bsz 8 with 80 strings, 9
 // passes of 209 us -> 4 of 213 us (12 bits with 4 low ones: 5 of 189 us; 14
 // bits, one workgroup of 1024 threads per CU: 3 of 490 us); 24 qubits bsz 64
-// with 48 strings, 3 passes of 6.7 -> 5.0 ms.  Held to 128 registers (four
+// with 48 strings, 3 passes of 6.7 -> 5.0 ms (203 us and 4.8 ms since a launch
+// needs less beside its groups).  Held to 128 registers (four
 // wavefronts per SIMD): with addresses in registers and the group's psi kept
 // beside the next one's the compiler took 218, and a pass 330 us.
 //
@@ -989,7 +990,7 @@ static PGPlan pg_build(int n, int m, const std::vector<uint32_t>& x, const std::
 }
 
 // The sets of a list of terms, kept for the next call with the same list (a
-// loop over one observable): planning 80 terms takes about 0.1 ms.  At most
+// loop over one observable): planning 80 terms takes about 0.05 ms.  At most
 // 64 lists; holds masks only, nothing of a state or a stream.
 static std::shared_ptr<const PGPlan> pg_plan(int n, int nterms, const uint64_t* xmask, const uint64_t* zmask) {
   struct Entry {
